@@ -88,6 +88,33 @@ __device__ __forceinline__ float sum_xor32(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+
+// Sum / maximum over the 64 lanes, the result in every lane: lane pairs i ^ 1,
+// i ^ 2 (quad permutes), then the mirrored lane within 8 and within 16 (each
+// lane of a quad / half-row holds the same partial by then, so the mirror
+// pairs the same partials as i ^ 4, i ^ 8), then rows i ^ 16 and halves i ^ 32
+// (permlane swaps).
+__device__ __forceinline__ float wave_sum(float v) {
+  v += dpp_move<0xB1>(v);
+  v += dpp_move<0x4E>(v);
+  v += dpp_move<0x141>(v);
+  v += dpp_move<0x140>(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return sum_xor32(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, dpp_move<0xB1>(v));
+  v = fmaxf(v, dpp_move<0x4E>(v));
+  v = fmaxf(v, dpp_move<0x141>(v));
+  v = fmaxf(v, dpp_move<0x140>(v));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return max_xor32(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+
 __device__ __forceinline__ float shfl_xor(float x, int m) {
   return __shfl_xor(x, m, 64);
 }

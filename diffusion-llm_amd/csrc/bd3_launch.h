@@ -125,7 +125,14 @@ struct SubsArgs {
   double keep;         // s / t
   const double* u;     // (rows, vocab) uniforms, or null: Philox4x32-10(seed, offset)
   uint64_t seed, offset;
+  // Few rows: `spread` workgroups dealt out over the masked rows, at most
+  // `slices` to a row, their results in ws (rows, slices) of kSubsSliceBytes;
+  // 0: one workgroup per row, which needs no workspace.
+  int spread, slices;
+  void* ws;
 };
+constexpr size_t kSubsSliceBytes = 512;
+constexpr int kSubsSpreadRows = 1024;  // most rows of a spread call
 
 struct GlueArgs {
   const void* x;       // (batch, seq, d) rows, fp32 or bf16

@@ -654,9 +654,24 @@ int bd3_kv_write(const void* k, const void* v, void* k_dst, void* v_dst, int32_t
   return hip_status(bd3::launch_kv_write(a, static_cast<hipStream_t>(stream)), "kv_write launch");
 }
 
-int bd3_subs_sample(const void* logits, int64_t ld, int32_t logits_fp32, const int64_t* xt,
-                    int64_t* out, int32_t rows, int32_t vocab, int32_t mask_index, double keep,
-                    const double* u, uint64_t seed, uint64_t offset, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// Slices a row of the sampling scan may be cut into (1: one workgroup per
+// row): each takes at least 2048 of the row's elements (one pair per thread),
+// and 16 of them put 16 rows on every CU; 24 measured the same (17.2 us a call
+// for one 16-token block). Above kSubsSpreadRows rows there is a workgroup for
+// every CU four times over without slices.
+constexpr int kSubsSpread = 512;  // workgroups of a spread call: two 1024-thread ones per CU
+int subs_slices(int32_t rows, int32_t vocab) {
+  if (rows > bd3::kSubsSpreadRows) return 1;
+  return std::max(1, std::min(vocab / 2048, 16));
+}
+
+int run_subs_sample(const void* logits, int64_t ld, int32_t logits_fp32, const int64_t* xt, int64_t* out,
+                    int32_t rows, int32_t vocab, int32_t mask_index, double keep, const double* u, uint64_t seed,
+                    uint64_t offset, int slices, void* workspace, void* stream) {
   if (rows < 0) return fail(BD3_EINVAL, "rows must be >= 0");
   if (vocab < 2) return fail(BD3_EINVAL, "vocab must be >= 2, got %d", vocab);
   if (mask_index < 0 || mask_index >= vocab)
@@ -679,7 +694,40 @@ int bd3_subs_sample(const void* logits, int64_t ld, int32_t logits_fp32, const i
   a.u = u;
   a.seed = seed;
   a.offset = offset;
+  a.slices = slices;
+  a.spread = slices > 1 ? std::max(kSubsSpread, (rows + 7) & ~7) : 0;
+  a.ws = workspace;
   return hip_status(bd3::launch_subs_sample(a, static_cast<hipStream_t>(stream)), "subs_sample launch");
+}
+
+}  // namespace
+
+extern "C" {
+
+int bd3_subs_sample(const void* logits, int64_t ld, int32_t logits_fp32, const int64_t* xt,
+                    int64_t* out, int32_t rows, int32_t vocab, int32_t mask_index, double keep,
+                    const double* u, uint64_t seed, uint64_t offset, void* stream) {
+  return run_subs_sample(logits, ld, logits_fp32, xt, out, rows, vocab, mask_index, keep, u, seed, offset, 1,
+                         nullptr, stream);
+}
+
+size_t bd3_subs_sample_workspace_bytes(int32_t rows, int32_t vocab) {
+  if (rows < 1 || vocab < 2) return 0;
+  const int s = subs_slices(rows, vocab);
+  return s > 1 ? (size_t)rows * s * bd3::kSubsSliceBytes : 0;
+}
+
+int bd3_subs_sample_ws(const void* logits, int64_t ld, int32_t logits_fp32, const int64_t* xt,
+                       int64_t* out, int32_t rows, int32_t vocab, int32_t mask_index, double keep,
+                       const double* u, uint64_t seed, uint64_t offset, void* workspace,
+                       size_t workspace_bytes, void* stream) {
+  const size_t need = bd3_subs_sample_workspace_bytes(rows, vocab);
+  if (workspace_bytes < need)
+    return fail(BD3_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
+  if (need > 0 && (workspace == nullptr || !aligned16(workspace)))
+    return fail(BD3_EINVAL, "workspace must be a 16-byte aligned device pointer");
+  return run_subs_sample(logits, ld, logits_fp32, xt, out, rows, vocab, mask_index, keep, u, seed, offset,
+                         need > 0 ? subs_slices(rows, vocab) : 1, workspace, stream);
 }
 
 namespace {

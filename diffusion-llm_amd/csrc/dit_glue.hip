@@ -77,33 +77,6 @@ __device__ __forceinline__ const char* elem(const void* base, int fp32, int64_t 
   return static_cast<const char*>(base) + i * (fp32 ? 4 : 2);
 }
 
-__device__ __forceinline__ float dpp_add(float v, int ctrl_sel) {
-  int t;
-  switch (ctrl_sel) {
-    case 0: t = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false); break;   // quad [1,0,3,2]
-    case 1: t = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false); break;   // quad [2,3,0,1]
-    case 2: t = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false); break;  // row_half_mirror
-    default: t = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false); break; // row_mirror
-  }
-  return v + __int_as_float(t);
-}
-
-// Sum over the 64 lanes, the total in every lane: lane pairs i ^ 1, i ^ 2
-// (quad permutes), then the mirrored lane within 8 and within 16 (each lane
-// of a quad / half-row holds the same partial by then, so the mirror pairs
-// the same partials as i ^ 4, i ^ 8), then rows i ^ 16 and halves i ^ 32
-// (permlane swaps).
-__device__ __forceinline__ float wave_sum(float v) {
-  v = dpp_add(v, 0);
-  v = dpp_add(v, 1);
-  v = dpp_add(v, 2);
-  v = dpp_add(v, 3);
-  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
-  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r32[0]) + __uint_as_float(r32[1]);
-}
-
 // The LayerNorm weight and the shift / scale of one row's batch index, as
 // raw loads: for rows of up to CH = 4 chunks per lane all of them are issued
 // with the row's own loads (PRE); longer rows load each chunk's vectors where

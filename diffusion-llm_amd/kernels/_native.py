@@ -54,6 +54,9 @@ SIGNATURES: dict[str, tuple] = {
     "bd3_kv_write": (ctypes.c_int, [_c_p, _c_p, _c_p, _c_p, _i32, _i32, _i32, _i32, _i64p, _c_p]),
     "bd3_subs_sample": (ctypes.c_int, [_c_p, ctypes.c_int64, _i32, _c_p, _c_p, _i32, _i32, _i32, ctypes.c_double,
                                        _c_p, ctypes.c_uint64, ctypes.c_uint64, _c_p]),
+    "bd3_subs_sample_workspace_bytes": (_sz, [_i32, _i32]),
+    "bd3_subs_sample_ws": (ctypes.c_int, [_c_p, ctypes.c_int64, _i32, _c_p, _c_p, _i32, _i32, _i32, ctypes.c_double,
+                                          _c_p, ctypes.c_uint64, ctypes.c_uint64, _c_p, _sz, _c_p]),
     "bd3_ln_modulate": (ctypes.c_int, [_c_p, _i32, _c_p, _i32, _c_p, _c_p, _i32, _c_p, _i32, _i32, _i32, _i32,
                                        _i64p, _f32, _c_p]),
     "bd3_gate_residual": (ctypes.c_int, [_c_p, _i32, _c_p, _i32, _c_p, _i32, _c_p, _i32, _i32, _i32, _i64p, _c_p]),

@@ -6,7 +6,7 @@ one denoising step of sample_bd3lm (sample/sampler.py:110-122): SUBS
 log-probs of the raw logits (model/subs.py:11-43), q = exp(log_probs) *
 (1 - s/t) with q[mask] = s/t, a Gumbel-max draw with float64 noise
 (sample_categorical, :11-34), and masked positions replaced by the draw.
-One bd3_subs_sample launch does it without writing any (rows, vocab)
+bd3_subs_sample_ws does it without writing any (rows, vocab)
 intermediate (the reference materialises the log-probs, the carry tensor,
 q, the uniforms and the noise, several of them in float64).
 
@@ -78,7 +78,9 @@ def subs_sample_step(
     else:
         gen = generator or default_stream()
         seed, offset = gen.seed, gen.next_offset()
-    check(lib().bd3_subs_sample(ptr(lg), lg.stride(0), 1 if lg.dtype == torch.float32 else 0, ptr(xt),
-                                ptr(out), rows, vocab, mask_index, float(keep), ptr(u), seed, offset,
-                                stream_of(lg)))
+    nbytes = lib().bd3_subs_sample_workspace_bytes(rows, vocab)
+    ws = torch.empty(nbytes, device=lg.device, dtype=torch.uint8) if nbytes else None
+    check(lib().bd3_subs_sample_ws(ptr(lg), lg.stride(0), 1 if lg.dtype == torch.float32 else 0, ptr(xt),
+                                   ptr(out), rows, vocab, mask_index, float(keep), ptr(u), seed, offset,
+                                   ptr(ws), nbytes, stream_of(lg)))
     return out.view(block.shape)

@@ -334,6 +334,19 @@ int bd3_subs_sample(const void* logits, int64_t ld, int32_t logits_fp32, const i
                     const double* u, uint64_t seed, uint64_t offset, void* stream);
 
 /*
+ * bd3_subs_sample with a caller-allocated workspace, which lets several
+ * workgroups share a row when there are few rows (a second, small launch then
+ * picks the token): the same tokens, up to the fp32 summation order of the
+ * row's exponentials. workspace_bytes >= bd3_subs_sample_workspace_bytes()
+ * (0: one workgroup per row is used; pass NULL / 0). No reference counterpart.
+ */
+size_t bd3_subs_sample_workspace_bytes(int32_t rows, int32_t vocab);
+int bd3_subs_sample_ws(const void* logits, int64_t ld, int32_t logits_fp32, const int64_t* xt,
+                       int64_t* out, int32_t rows, int32_t vocab, int32_t mask_index, double keep,
+                       const double* u, uint64_t seed, uint64_t offset, void* workspace,
+                       size_t workspace_bytes, void* stream);
+
+/*
  * modulate(LN(x), shift, scale) of a DiT block's pre-norm (weight-only
  * LayerNorm, model/modules.py:243-288; modulate, :778-788; call sites in
  * DiTBlock.forward, :537-568), one pass over x:

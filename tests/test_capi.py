@@ -407,3 +407,20 @@ def test_fused_glue_validation(lib):
     expect_einval(fu(yf=3), "dtype flags")
     expect_einval(fu(eps=float("nan")), "eps")
     expect_einval(fu(st=_i64([768 * 16, 768, 768 * 6, 768 * 16, 768, 768 * 16, 769, 768 * 16, 768])), "stride[6]")
+
+
+def test_subs_sample_workspace_validation(lib):
+    """The workspace form: sized by rows and vocabulary, refused when it is
+    too small, missing or misaligned; none is needed where a row is not cut."""
+    p = 1 << 20  # never dereferenced: the call is refused first
+    size = lib.bd3_subs_sample_workspace_bytes
+    assert size(16, 50258) == 16 * 16 * 512 and size(1024, 4096) == 1024 * 2 * 512
+    assert size(16, 4095) == size(1025, 50258) == size(0, 50258) == size(16, 1) == 0
+
+    def call(ws, nbytes, rows=16, vocab=50258, mask=50257):
+        return lib.bd3_subs_sample_ws(p, vocab, 0, p, p, rows, vocab, mask, 0.5, None, 0, 0, ws, nbytes, None)
+
+    need = size(16, 50258)
+    for ws, nbytes in ((p, need - 1), (None, need), (p + 8, need)):
+        assert call(ws, nbytes) == _native.BD3_EINVAL and "workspace" in _native.last_error()
+    assert call(p, need, mask=50258) == _native.BD3_EINVAL and "mask_index" in _native.last_error()

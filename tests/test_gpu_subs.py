@@ -106,3 +106,64 @@ def test_near_ties_resolved_exactly(cuda, vocab, mask):
     assert want.tolist() == [b, b, min(a, b), mask]
     got = subs_sample_step(logits.to(cuda), xt.to(cuda), mask, keep, u=u.to(cuda))
     assert torch.equal(got.cpu(), want)
+
+
+def one_workgroup_per_row(logits, xt, mask, keep, u=None, seed=0, offset=0):
+    """bd3_subs_sample itself: no workspace, so a row is never cut into slices."""
+    from kernels._native import check, lib, ptr, stream_of
+    out = torch.empty_like(xt)
+    check(lib().bd3_subs_sample(ptr(logits), logits.stride(0), int(logits.dtype == torch.float32), ptr(xt), ptr(out),
+                                logits.shape[0], logits.shape[1], mask, float(keep), ptr(u), seed, offset,
+                                stream_of(logits)))
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,vocab,mask,extra,dtype", [
+    (1, 4095, 0, 0, torch.bfloat16),        # one slice (two need 4096), [MASK] first
+    (1, 4096, 4095, 0, torch.bfloat16),     # two slices
+    (9, 4099, 4098, 0, torch.bfloat16),     # odd rows start inside an element pair and off a 4-byte boundary
+    (64, 6145, 2048, 1, torch.bfloat16),    # [MASK] at the start of a slice, even row stride
+    (65, 8191, 8190, 3, torch.float32),     # rows cross a group of 64
+    (200, 50258, 50257, 0, torch.bfloat16),  # more masked rows than half the workgroups: one slice each, or two
+    (1024, 4096, 17, 0, torch.bfloat16),    # the most rows that are spread
+    (1025, 4096, 17, 0, torch.bfloat16),    # one workgroup per row
+])
+@pytest.mark.parametrize("masked", [1.0, 0.3])
+def test_slices_match_oracle(cuda, rows, vocab, mask, extra, dtype, masked):
+    """The row cut into slices, the masked rows dealt out over the workgroups
+    and the candidates' second pass draw the oracle's tokens; so does the
+    entry point without a workspace."""
+    print(f"subs_sample slices rows={rows} vocab={vocab} masked={masked}", flush=True)
+    wide, xt = make(rows, vocab + extra, mask, dtype, seed=rows + vocab, masked_frac=masked)
+    wide, xt = wide.to(cuda), xt.clamp(max=vocab - 1).to(cuda)
+    logits = wide[:, :vocab]
+    gen = PhiloxStream(seed=rows * 7919 + vocab)
+    got = subs_sample_step(logits, xt, mask, 0.25, generator=gen)
+    want = orc.sample_step(logits.cpu(), xt.cpu(), mask, 0.25, orc.philox_uniforms(gen.seed, 0, rows, vocab))
+    assert torch.equal(got.cpu(), want)
+    assert torch.equal(one_workgroup_per_row(logits, xt, mask, 0.25, seed=gen.seed).cpu(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_without_usable_bounds_match_oracle(cuda, dtype):
+    """Rows that the pruning bounds cannot narrow are evaluated element by
+    element: [MASK]'s logit above the others by more than its bias (every
+    exponential may underflow), and every ratio equal (more contenders than
+    the candidate list holds; the first index wins)."""
+    rows, vocab, mask = 4, 50258, 50257
+    g = torch.Generator().manual_seed(3)
+    logits = torch.randn(rows, vocab, generator=g)
+    logits[0, mask] = 3e6
+    logits[1, mask] = 1e6
+    logits[2] = 0.5
+    logits = logits.to(dtype)
+    xt = torch.full((rows,), mask, dtype=torch.int64)
+    u = torch.rand(rows, vocab, dtype=torch.float64, generator=g)
+    u[2] = 0.25
+    for keep in (0.0, 0.5):
+        want = orc.sample_step(logits, xt, mask, keep, u)
+        args = [t.to(cuda) for t in (logits, xt)]
+        assert torch.equal(subs_sample_step(*args, mask, keep, u=u.to(cuda)).cpu(), want)
+        assert torch.equal(one_workgroup_per_row(*args, mask, keep, u=u.to(cuda)).cpu(), want)
