@@ -147,6 +147,7 @@ struct GlueArgs {
   int rows, seq, d;
   int64_t sx_b, sx_s, sm_b, sy_b, sy_s, so_b, so_s, sxo_b, sxo_s;  // element strides
   float eps;
+  int wave_rows, wg_threads;  // set at the launch: rows per wave, threads per workgroup
 };
 
 hipError_t launch_attn_fwd(const FwdArgs& a, hipStream_t stream);

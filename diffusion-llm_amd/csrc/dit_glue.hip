@@ -11,14 +11,17 @@
 //     promoted dtype of y and the vectors (bf16 if both are bf16, every op
 //     rounded, as eager bf16 tensor ops; fp32 otherwise), optionally rounded
 //     to bf16 for the next matmul (what autocast does at its input).
-//   One wavefront per row (64 lanes x 16-byte chunks); the row is read from
-//   HBM once and kept in registers (d_model <= 4096). Every load of a row and
-//   of its vectors is issued before the first use (loads whose dtype is a
-//   run-time flag are issued as raw 16-byte pairs and decoded later, so no
-//   branch separates them), and the row sums are reduced with DPP and
-//   permlane swaps instead of LDS permutes.
-// gate_residual_ln_modulate_kernel: the two fused (a residual update, then
-//   the next sublayer's LayerNorm + modulate of the updated row).
+//   FUSED: of the updated residual row x + gate * y, which is stored too.
+//   Bound by HBM: a row is read once into registers (d_model <= 4096), its sums
+//   are reduced with DPP and permlane swaps. Dtypes are template arguments and
+//   every load and store of a wave is one contiguous piece (4-element chunks: 1
+//   KB of fp32, 512 B of bf16); with 8-element chunks and run-time dtypes a
+//   fp32 load spanned twice its bytes, a bf16 one was issued twice, half the
+//   lanes of a 768-wide row were idle and every row reloaded its vectors (6 KB
+//   against the row's own 4.5). 8 x 2048 x 768, fp32 x, bf16 result: 17.2 ->
+//   12.9 us (5.9 TB/s); FUSED 37.6 -> 31.1 us (4.9 TB/s); bf16 x: 16.7 -> 11.8
+//   and 29.3 -> 23.4 us; 4096 x 2048 fp32: 15.9 -> 12.4 and 26.4 -> 23.5 us; 1024
+//   x 4096: 12.7 -> 9.4 and 17.3 -> 13.6 us.
 // gate_residual_kernel: x + gate * y (the residual updates of
 //   DiTBlock.forward, :560-566): gate * y in the promoted dtype of gate and y,
 //   then the add in the promoted dtype of x and that product; bit-exact with
@@ -77,168 +80,237 @@ __device__ __forceinline__ const char* elem(const void* base, int fp32, int64_t 
   return static_cast<const char*>(base) + i * (fp32 ? 4 : 2);
 }
 
-// The LayerNorm weight and the shift / scale of one row's batch index, as
-// raw loads: for rows of up to CH = 4 chunks per lane all of them are issued
-// with the row's own loads (PRE); longer rows load each chunk's vectors where
-// they are used (registers go to the row).
-template <int CH, bool PRE = (CH <= 4)>
-struct ModVecs {
-  Raw8 w[PRE ? CH : 1], sh[PRE ? CH : 1], sc[PRE ? CH : 1];
-  const char* shr;
-  const char* scr;
-  __device__ __forceinline__ ModVecs(const GlueArgs& a, int b, int lane) {
-    shr = elem(a.shift, a.m_fp32, (int64_t)b * a.sm_b);
-    scr = elem(a.scale, a.m_fp32, (int64_t)b * a.sm_b);
-    if constexpr (PRE) {
-      const int nch = a.d >> 3;
+// 4 consecutive elements as loaded: fp32 (16 bytes) or bf16 (8 bytes).
+template <bool F32>
+struct Raw4;
+template <>
+struct Raw4<true> {
+  u32x4 v;
+  __device__ __forceinline__ void load(const void* p) { v = ld16(p); }
+  __device__ __forceinline__ void get(float (&f)[4]) const {
 #pragma unroll
-      for (int k = 0; k < CH; ++k) {
-        const int c = imin(lane + 64 * k, nch - 1);  // lanes past the row repeat its last chunk
-        w[k] = ld_raw8(elem(a.weight, a.w_fp32, 8 * c), a.w_fp32);
-        sh[k] = ld_raw8(elem(shr, a.m_fp32, 8 * c), a.m_fp32);
-        sc[k] = ld_raw8(elem(scr, a.m_fp32, 8 * c), a.m_fp32);
-      }
-    }
-  }
-  __device__ __forceinline__ void chunk(const GlueArgs& a, int k, int c, float (&w8)[8], float (&sh8)[8],
-                                        float (&sc8)[8]) const {
-    if constexpr (PRE) {
-      unpack8(w[k], a.w_fp32, w8);
-      unpack8(sh[k], a.m_fp32, sh8);
-      unpack8(sc[k], a.m_fp32, sc8);
-    } else {
-      load8(elem(a.weight, a.w_fp32, 8 * c), a.w_fp32, w8);
-      load8(elem(shr, a.m_fp32, 8 * c), a.m_fp32, sh8);
-      load8(elem(scr, a.m_fp32, 8 * c), a.m_fp32, sc8);
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t w = v[k];
+      f[k] = __uint_as_float(w);
     }
   }
 };
+template <>
+struct Raw4<false> {
+  u32x2 v;
+  __device__ __forceinline__ void load(const void* p) { v = *static_cast<const u32x2*>(p); }
+  __device__ __forceinline__ void get(float (&f)[4]) const {
+    const uint32_t l = v[0], h = v[1];
+    f[0] = __uint_as_float(l << 16);
+    f[1] = __uint_as_float(l & 0xffff0000u);
+    f[2] = __uint_as_float(h << 16);
+    f[3] = __uint_as_float(h & 0xffff0000u);
+  }
+};
 
-// LayerNorm statistics of a row held in registers (v: CH 16-byte chunks per
-// lane, zero past the row), then modulate with the row's vectors and store
-// it. x_fp32: the row's dtype (the LayerNorm output is rounded back to it).
-template <int CH, class MV>
-__device__ __forceinline__ void ln_modulate_row(const GlueArgs& a, int b, int s, int lane,
-                                                const float (&v)[CH][8], const MV& mv, bool x_fp32) {
+__device__ __forceinline__ void store4(void* p, bool fp32, const float (&v)[4]) {
+  if (fp32)
+    *static_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+  else
+    *static_cast<bf16x4*>(p) = to_bf16x4(v[0], v[1], v[2], v[3]);
+}
+
+// modulate(LN(row), shift, scale), with FUSED of the updated residual row
+// x + gate * y (gate_residual_kernel's dtypes and roundings), which is stored
+// too: one launch and one read of the residual instead of two of each
+// (DiTBlock.forward, model/modules.py:560-566 then the next sublayer's
+// :537-568). out_x may alias x (a wave has read its row before it writes it,
+// and no other wave reads it).
+//
+// A wave owns `a.wave_rows` consecutive rows; lane l holds the 4-element chunks
+// l, l + 64, ... of a row, so every load and store of a wave is one contiguous
+// piece. CH: chunks per lane (d_model <= 256 * CH). Rows of up to 4 chunks per
+// lane keep the gain, 1 + scale and shift (and the gate) in registers from row
+// to row and request the next row before they work on the current one; longer
+// rows load them per row. XF / MF / YF: x, the vectors, y in fp32.
+template <int CH, bool XF, bool MF, bool YF, bool FUSED>
+__global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
 #pragma clang fp contract(off)  // separate products and sums, as the eager ops
-  const int D = a.d;
-  const int nch = D >> 3;
-  float sum = 0.f;
+  constexpr bool KEEP = CH <= 4;
+  constexpr bool kGyBf16 = !MF && !YF;
+  constexpr bool kRowF32 = FUSED ? XF || MF || YF : XF;  // dtype of the row that is normalised
+  constexpr bool kModBf16 = !kRowF32 && !MF;             // modulate in bf16 iff the row and the vectors are
+  const int lane = wi_x() & 63;
+  const int wave = wave_uniform((int)(wg_x() * (a.wg_threads >> 6) + (wi_x() >> 6)));
+  const int r0 = wave * a.wave_rows;
+  const int r1 = imin(a.rows, r0 + a.wave_rows);
+  if (r0 >= r1) return;
+  const int nch = a.d >> 2;
+  const float d_inv = (float)a.d;
+  int col[CH];  // first element of the lane's chunk k (lanes past the row repeat its last chunk)
 #pragma unroll
-  for (int k = 0; k < CH; ++k)
+  for (int k = 0; k < CH; ++k) col[k] = 4 * imin(lane + 64 * k, nch - 1);
+
+  auto x_row = [&](int b, int s) { return elem(a.x, XF, (int64_t)b * a.sx_b + (int64_t)s * a.sx_s); };
+  auto y_row = [&](int b, int s) { return elem(a.y, YF, (int64_t)b * a.sy_b + (int64_t)s * a.sy_s); };
+  Raw4<XF> xr[CH];
+  Raw4<YF> yr[FUSED ? CH : 1];
+  auto load_row = [&](int b, int s) {
+    const char* xp = x_row(b, s);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) sum += v[k][e];
-  const float mean = wave_sum(sum) / (float)D;
-  float sq = 0.f;
+    for (int k = 0; k < CH; ++k) xr[k].load(xp + col[k] * (XF ? 4 : 2));
+    if constexpr (FUSED) {
+      const char* yp = y_row(b, s);
 #pragma unroll
-  for (int k = 0; k < CH; ++k)
-    if (lane + 64 * k < nch) {
+      for (int k = 0; k < CH; ++k) yr[k].load(yp + col[k] * (YF ? 4 : 2));
+    }
+  };
+  int b = r0 / a.seq, s = r0 - b * a.seq;
+  load_row(b, s);
+
+  // gain; 1 + scale (rounded to the vectors' dtype: a Python scalar does not promote); shift; gate
+  constexpr int KV = KEEP ? CH : 1;
+  float w[KV][4], t[KV][4], sh[KV][4];
+  Raw4<MF> gate[FUSED && KEEP ? CH : 1];
+  auto load_w = [&](int k, float (&f)[4]) {
+    if (a.w_fp32) {
+      Raw4<true> r;
+      r.load(elem(a.weight, 1, col[k]));
+      r.get(f);
+    } else {
+      Raw4<false> r;
+      r.load(elem(a.weight, 0, col[k]));
+      r.get(f);
+    }
+  };
+  auto one_plus = [&](const Raw4<MF>& r, float (&f)[4]) {
+    r.get(f);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float dlt = v[k][e] - mean;
-        sq += dlt * dlt;
+    for (int e = 0; e < 4; ++e) f[e] = MF ? 1.f + f[e] : rbf(1.f + f[e]);
+  };
+  auto load_vectors = [&](int bb) {
+    Raw4<MF> rt[KV], rs[KV];
+#pragma unroll
+    for (int k = 0; k < KV; ++k) {
+      rt[k].load(elem(a.scale, MF, (int64_t)bb * a.sm_b + col[k]));
+      rs[k].load(elem(a.shift, MF, (int64_t)bb * a.sm_b + col[k]));
+      if constexpr (FUSED) gate[k].load(elem(a.gate, MF, (int64_t)bb * a.sm_b + col[k]));
+    }
+#pragma unroll
+    for (int k = 0; k < KV; ++k) {
+      one_plus(rt[k], t[k]);
+      rs[k].get(sh[k]);
+    }
+  };
+  // Rows of more than 4 chunks: requested with the row, decoded where they are
+  // used. The gain's dtype is a run-time flag: two 8-byte loads (the same 8
+  // bytes twice for bf16) instead of a branch that would wait for its load.
+  constexpr int RV = KEEP ? 1 : CH;
+  Raw4<MF> vt[RV], vs[RV], vg[FUSED ? RV : 1];
+  u32x2 wlo[RV], whi[RV];
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int k = 0; k < CH; ++k) load_w(k, w[k]);
+    load_vectors(b);
+  } else {
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      if constexpr (FUSED) vg[k].load(elem(a.gate, MF, (int64_t)b * a.sm_b + col[k]));
+      const char* wp = elem(a.weight, a.w_fp32, col[k]);
+      wlo[k] = *reinterpret_cast<const u32x2*>(wp);
+      whi[k] = *reinterpret_cast<const u32x2*>(wp + (a.w_fp32 ? 8 : 0));
+      vt[k].load(elem(a.scale, MF, (int64_t)b * a.sm_b + col[k]));
+      vs[k].load(elem(a.shift, MF, (int64_t)b * a.sm_b + col[k]));
+    }
+  }
+
+  for (int row = r0;;) {
+    // the row's values (zero past its end); with FUSED the updated residual, stored
+    float v[CH][4];
+    if constexpr (FUSED) {
+      char* xo = const_cast<char*>(elem(a.out_x, kRowF32, (int64_t)b * a.sxo_b + (int64_t)s * a.sxo_s));
+#pragma unroll
+      for (int k = 0; k < CH; ++k) {
+        float xv[4], yv[4], gv[4];
+        xr[k].get(xv);
+        yr[k].get(yv);
+        if constexpr (KEEP) {
+          gate[k].get(gv);
+        } else {
+          vg[k].get(gv);
+        }
+        const bool in = lane + 64 * k < nch;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float gy = gv[e] * yv[e];
+          if (kGyBf16) gy = rbf(gy);
+          const float o = xv[e] + gy;
+          v[k][e] = in ? (kRowF32 ? o : rbf(o)) : 0.f;
+        }
+        if (in) store4(xo + (int64_t)col[k] * (kRowF32 ? 4 : 2), kRowF32, v[k]);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < CH; ++k) {
+        xr[k].get(v[k]);
+        const bool in = lane + 64 * k < nch;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[k][e] = in ? v[k][e] : 0.f;
       }
     }
-  const float inv = rsqrtf(wave_sum(sq) / (float)D + a.eps);
-
-  const bool mod_bf16 = !x_fp32 && !a.m_fp32;  // modulate in bf16 iff y and the vectors are bf16
-  char* outr = const_cast<char*>(elem(a.out, a.out_fp32, (int64_t)b * a.so_b + (int64_t)s * a.so_s));
-#pragma unroll
-  for (int k = 0; k < CH; ++k) {
-    const int c = lane + 64 * k;
-    if (c >= nch) break;
-    float w[8], sh[8], sc[8], o[8];
-    mv.chunk(a, k, c, w, sh, sc);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float y = (w[e] * (v[k][e] - mean)) * inv;
-      if (!x_fp32) y = rbf(y);  // .to(original dtype)
-      // 1 + scale keeps scale's dtype (a Python scalar does not promote)
-      const float t = a.m_fp32 ? 1.f + sc[e] : rbf(1.f + sc[e]);
-      o[e] = mod_bf16 ? rbf(rbf(y * t) + sh[e]) : y * t + sh[e];
+    const int nrow = row + 1;
+    int nb = b, ns = s + 1;
+    if (ns == a.seq) {
+      ns = 0;
+      ++nb;
     }
-    store8(outr + (int64_t)8 * c * (a.out_fp32 ? 4 : 2), a.out_fp32, o);
-  }
-}
+    if constexpr (KEEP)
+      if (nrow < r1) load_row(nb, ns);
 
-// Chunk k of a lane, zero past the row.
-template <int CH>
-__device__ __forceinline__ void unpack_row(const Raw8 (&r)[CH], int fp32, int lane, int nch, float (&v)[CH][8]) {
+    float sum = 0.f;
 #pragma unroll
-  for (int k = 0; k < CH; ++k) {
-    unpack8(r[k], fp32, v[k]);
-    const bool in = lane + 64 * k < nch;
+    for (int k = 0; k < CH; ++k)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[k][e] = in ? v[k][e] : 0.f;
-  }
-}
-
-// CH: 16-byte chunks (8 elements) of the row held per lane; the row is read
-// from HBM once into registers (d_model <= 512 * CH).
-template <int CH>
-__global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
-  const int row = wg_x() * 4 + (wi_x() >> 6);
-  if (row >= a.rows) return;
-  const int lane = wi_x() & 63;
-  const int b = row / a.seq, s = row - b * a.seq;
-  const int nch = a.d >> 3;
-  const void* xr = elem(a.x, a.x_fp32, (int64_t)b * a.sx_b + (int64_t)s * a.sx_s);
-  Raw8 xraw[CH];
+      for (int e = 0; e < 4; ++e) sum += v[k][e];
+    const float mean = wave_sum(sum) / d_inv;
+    float sq = 0.f;
 #pragma unroll
-  for (int k = 0; k < CH; ++k) xraw[k] = ld_raw8(elem(xr, a.x_fp32, 8 * imin(lane + 64 * k, nch - 1)), a.x_fp32);
-  const ModVecs<CH> mv(a, b, lane);
-  float v[CH][8];
-  unpack_row<CH>(xraw, a.x_fp32, lane, nch, v);
-  ln_modulate_row<CH>(a, b, s, lane, v, mv, a.x_fp32);
-}
-
-// The residual update x + gate * y (gate_residual_kernel's dtypes and
-// roundings) followed by modulate(LN(.)) of the updated row, which stays in
-// registers: one launch and one read of the residual instead of two of each
-// (DiTBlock.forward, model/modules.py:560-566 then the next sublayer's
-// :537-568). out_x may alias x (each lane reads its chunks before it writes
-// them).
-template <int CH>
-__global__ __launch_bounds__(256) void gate_residual_ln_modulate_kernel(GlueArgs a) {
-#pragma clang fp contract(off)  // gate * y rounded before the add, as the eager ops
-  const int row = wg_x() * 4 + (wi_x() >> 6);
-  if (row >= a.rows) return;
-  const int lane = wi_x() & 63;
-  const int b = row / a.seq, s = row - b * a.seq;
-  const int nch = a.d >> 3;
-  const bool gy_bf16 = !a.m_fp32 && !a.y_fp32;
-  const bool res_bf16 = !a.x_fp32 && gy_bf16;  // dtype of x + gate * y
-  const void* xr = elem(a.x, a.x_fp32, (int64_t)b * a.sx_b + (int64_t)s * a.sx_s);
-  const void* gr = elem(a.gate, a.m_fp32, (int64_t)b * a.sm_b);
-  const void* yr = elem(a.y, a.y_fp32, (int64_t)b * a.sy_b + (int64_t)s * a.sy_s);
-  char* xo = const_cast<char*>(elem(a.out_x, !res_bf16, (int64_t)b * a.sxo_b + (int64_t)s * a.sxo_s));
-  Raw8 xraw[CH], graw[CH], yraw[CH];
+    for (int k = 0; k < CH; ++k) {
+      const bool in = lane + 64 * k < nch;
 #pragma unroll
-  for (int k = 0; k < CH; ++k) {
-    const int c = imin(lane + 64 * k, nch - 1);
-    xraw[k] = ld_raw8(elem(xr, a.x_fp32, 8 * c), a.x_fp32);
-    graw[k] = ld_raw8(elem(gr, a.m_fp32, 8 * c), a.m_fp32);
-    yraw[k] = ld_raw8(elem(yr, a.y_fp32, 8 * c), a.y_fp32);
-  }
-  const ModVecs<CH> mv(a, b, lane);
-  float v[CH][8];
-#pragma unroll
-  for (int k = 0; k < CH; ++k) {
-    const int c = lane + 64 * k;
-    float xv[8], gv[8], yv[8];
-    unpack8(xraw[k], a.x_fp32, xv);
-    unpack8(graw[k], a.m_fp32, gv);
-    unpack8(yraw[k], a.y_fp32, yv);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float gy = gv[e] * yv[e];
-      if (gy_bf16) gy = rbf(gy);
-      const float o = xv[e] + gy;
-      v[k][e] = c < nch ? (res_bf16 ? rbf(o) : o) : 0.f;  // the value the residual store keeps
+      for (int e = 0; e < 4; ++e) {
+        v[k][e] -= mean;
+        const float dd = v[k][e] * v[k][e];
+        sq += in ? dd : 0.f;
+      }
     }
-    if (c < nch) store8(xo + (int64_t)8 * c * (res_bf16 ? 2 : 4), !res_bf16, v[k]);
+    const float inv = rsqrtf(wave_sum(sq) / d_inv + a.eps);
+    char* outr = const_cast<char*>(elem(a.out, a.out_fp32, (int64_t)b * a.so_b + (int64_t)s * a.so_s));
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      float wk[4], tk[4], shk[4], o[4];
+      if constexpr (!KEEP) {
+        float wb[4];
+        Raw4<false>{wlo[k]}.get(wb);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t f = e < 2 ? wlo[k][e] : whi[k][e - 2];
+          wk[e] = a.w_fp32 ? __uint_as_float(f) : wb[e];
+        }
+        one_plus(vt[k], tk);
+        vs[k].get(shk);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float y = ((KEEP ? w[KEEP ? k : 0][e] : wk[e]) * v[k][e]) * inv;
+        if (!kRowF32) y = rbf(y);  // .to(original dtype)
+        const float te = KEEP ? t[KEEP ? k : 0][e] : tk[e], se = KEEP ? sh[KEEP ? k : 0][e] : shk[e];
+        o[e] = kModBf16 ? rbf(rbf(y * te) + se) : y * te + se;
+      }
+      if (lane + 64 * k < nch) store4(outr + (int64_t)col[k] * (a.out_fp32 ? 4 : 2), a.out_fp32, o);
+    }
+    if (!KEEP || nrow >= r1) break;
+    if constexpr (KEEP)
+      if (nb != b) load_vectors(nb);
+    row = nrow;
+    b = nb;
+    s = ns;
   }
-  ln_modulate_row<CH>(a, b, s, lane, v, mv, !res_bf16);
 }
 
 // 4 consecutive elements at p: fp32 (16 bytes) or bf16 (8 bytes), the dtype
@@ -313,38 +385,65 @@ __global__ __launch_bounds__(256) void gate_residual_kernel(GlueArgs a) {
 
 }  // namespace
 
-hipError_t launch_ln_modulate(const GlueArgs& a, hipStream_t stream) {
+namespace {
+
+template <int CH, bool FUSED>
+void launch_rows_ch(const GlueArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
+#define BD3_ROWS(XF, MF, YF) hipLaunchKernelGGL((ln_modulate_kernel<CH, XF, MF, YF, FUSED>), grid, block, 0, stream, a)
+  const int t = (a.x_fp32 ? 4 : 0) | (a.m_fp32 ? 2 : 0) | (FUSED && a.y_fp32 ? 1 : 0);
+  switch (t) {
+    case 0: BD3_ROWS(false, false, false); break;
+    case 2: BD3_ROWS(false, true, false); break;
+    case 4: BD3_ROWS(true, false, false); break;
+    case 6: BD3_ROWS(true, true, false); break;
+    default:
+      if constexpr (FUSED) {
+        if (t == 1) BD3_ROWS(false, false, true);
+        if (t == 3) BD3_ROWS(false, true, true);
+        if (t == 5) BD3_ROWS(true, false, true);
+        if (t == 7) BD3_ROWS(true, true, true);
+      }
+  }
+#undef BD3_ROWS
+}
+
+template <bool FUSED>
+hipError_t launch_rows(GlueArgs a, hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
-  const dim3 grid((unsigned)((a.rows + 3) / 4));
-  const int ch = (a.d / 8 + 63) / 64;  // chunks per lane
+  const int ch = (a.d / 4 + 63) / 64;  // 4-element chunks per lane
+  if (ch > 16) return hipErrorInvalidValue;  // d_model > 4096: rejected by the C ABI
+  // Rows per wave: enough waves to keep 8 per SIMD (8192 over 1024 SIMDs), then
+  // up to 8 rows each, so that the vectors are loaded once for them and the
+  // next row is on its way. 8 x 2048 rows x 768 (fp32 residual): fused 31.1 us at
+  // 2 rows a wave, 32.5 at 4, 34.4 at 8, 31.9 at 1; alone 12.9 / 12.8 / 13.6 /
+  // 13.8. Few rows take one-wave workgroups, which spread over all CUs.
+  a.wave_rows = ch <= 4 ? imin(imax(a.rows / 8192, 1), 8) : 1;
+  const int waves = (a.rows + a.wave_rows - 1) / a.wave_rows;
+  a.wg_threads = waves <= 1024 ? 64 : 256;
+  const dim3 block(a.wg_threads), grid((unsigned)((waves * 64 + a.wg_threads - 1) / a.wg_threads));
   if (ch <= 1)
-    hipLaunchKernelGGL(ln_modulate_kernel<1>, grid, dim3(256), 0, stream, a);
+    launch_rows_ch<1, FUSED>(a, grid, block, stream);
   else if (ch <= 2)
-    hipLaunchKernelGGL(ln_modulate_kernel<2>, grid, dim3(256), 0, stream, a);
+    launch_rows_ch<2, FUSED>(a, grid, block, stream);
+  else if (ch <= 3)
+    launch_rows_ch<3, FUSED>(a, grid, block, stream);
   else if (ch <= 4)
-    hipLaunchKernelGGL(ln_modulate_kernel<4>, grid, dim3(256), 0, stream, a);
+    launch_rows_ch<4, FUSED>(a, grid, block, stream);
+  else if (ch <= 6)
+    launch_rows_ch<6, FUSED>(a, grid, block, stream);
   else if (ch <= 8)
-    hipLaunchKernelGGL(ln_modulate_kernel<8>, grid, dim3(256), 0, stream, a);
+    launch_rows_ch<8, FUSED>(a, grid, block, stream);
   else
-    return hipErrorInvalidValue;  // d_model > 4096: rejected by the C ABI
+    launch_rows_ch<16, FUSED>(a, grid, block, stream);
   return hipGetLastError();
 }
 
+}  // namespace
+
+hipError_t launch_ln_modulate(const GlueArgs& a, hipStream_t stream) { return launch_rows<false>(a, stream); }
+
 hipError_t launch_gate_residual_ln_modulate(const GlueArgs& a, hipStream_t stream) {
-  if (a.rows == 0) return hipSuccess;
-  const dim3 grid((unsigned)((a.rows + 3) / 4));
-  const int ch = (a.d / 8 + 63) / 64;  // chunks per lane
-  if (ch <= 1)
-    hipLaunchKernelGGL(gate_residual_ln_modulate_kernel<1>, grid, dim3(256), 0, stream, a);
-  else if (ch <= 2)
-    hipLaunchKernelGGL(gate_residual_ln_modulate_kernel<2>, grid, dim3(256), 0, stream, a);
-  else if (ch <= 4)
-    hipLaunchKernelGGL(gate_residual_ln_modulate_kernel<4>, grid, dim3(256), 0, stream, a);
-  else if (ch <= 8)
-    hipLaunchKernelGGL(gate_residual_ln_modulate_kernel<8>, grid, dim3(256), 0, stream, a);
-  else
-    return hipErrorInvalidValue;  // d_model > 4096: rejected by the C ABI
-  return hipGetLastError();
+  return launch_rows<true>(a, stream);
 }
 
 hipError_t launch_gate_residual(const GlueArgs& a, hipStream_t stream) {

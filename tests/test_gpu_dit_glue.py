@@ -105,3 +105,32 @@ def test_gate_residual_ln_modulate_matches_two_calls(cuda, xd, md, yd, od, B, S,
     want_h3 = ln_modulate(want_x, w, fin[:, 0], fin[:, 1], out_dtype=od)
     _, got_h3 = gate_residual_ln_modulate(x, g, y, w, fin[:, 0], fin[:, 1], out_dtype=od)
     assert torch.equal(got_h3, want_h3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("xd", [F32, BF])
+# 16383 rows: one per wave; 16384 and 24579: two and three, an odd sequence
+# length, so a wave's rows lie in two batch entries; 65537: eight, and a last
+# wave with one. d = 64, 264, 768, 1016: one to four chunks a lane, the last
+# chunk of 264 and 1016 not in every lane.
+@pytest.mark.parametrize("B,S,D", [(3, 5461, 768), (4, 4096, 264), (3, 8193, 1016), (65537, 1, 64)])
+def test_several_rows_per_wave(cuda, xd, B, S, D):
+    from kernels.dit_glue import gate_residual_ln_modulate
+    print(f"rows per wave x={xd} shape=({B},{S},{D})", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(21)
+    x, y = (torch.randn(B, S, D, generator=g, device=cuda) for _ in range(2))
+    x, y = (2 * x + 0.3).to(xd), y.to(BF)
+    ada = (0.5 * torch.randn(B, 6, 1, D, generator=g, device=cuda)).to(BF)
+    gate, sh, sc = ada[:, 2], ada[:, 3], ada[:, 4]
+    w = 1 + 0.2 * torch.randn(D, generator=g, device=cuda)
+    want_x = ref_gate(x, gate[:, 0], y)
+    got_x, got_h = gate_residual_ln_modulate(x, gate, y, w, sh, sc, out_dtype=BF)
+    assert torch.equal(got_x, want_x)
+    assert torch.equal(got_h, ln_modulate(want_x, w, sh, sc, out_dtype=BF))
+    # test_ln_modulate's bound: one bf16 ulp per rounding of the magnitudes entering the last add
+    h = ref_layer_norm(want_x, w).float()
+    want = (h.to(xd) * (1 + sc) + sh).to(BF).float()
+    mag = (h * (1 + sc.float())).abs() + sh.float().abs()
+    diff = (got_h.float() - want).abs()
+    assert (diff <= 3 * 2.0 ** -7 * mag + 1e-30).all(), float((diff / (mag + 1e-30)).max())
+    assert (diff > 0).float().mean() < 0.01, float((diff > 0).float().mean())
