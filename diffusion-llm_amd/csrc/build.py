@@ -1,11 +1,11 @@
 """Build libbd3attn.so for gfx950 with hipcc (no GPU needed: hipcc
-cross-compiles the device code).
+cross-compiles the device code) and bd3_host.so, the CPython extension that
+prepares the kernels' calls, with g++ against the installed torch.
 
     python diffusion-llm_amd/csrc/build.py [--jobs N] [--verbose]
 
-Sources: every *.hip file in this directory. Output:
-diffusion-llm_amd/lib/libbd3attn.so (git-ignored; it travels to the GPU box
-with the working tree).
+Sources: every *.hip file in this directory, and host_calls.cpp. Output:
+diffusion-llm_amd/lib/libbd3attn.so and bd3_host.so (git-ignored).
 """
 from __future__ import annotations
 
@@ -15,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent
@@ -22,6 +23,7 @@ PKG = CSRC.parent
 REPO = PKG.parent
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libbd3attn.so"
+HOST = LIB_DIR / "bd3_host.so"
 OBJ_DIR = PKG / "_build"
 
 ARCH = "gfx950"
@@ -71,8 +73,30 @@ def _compile(src: Path, verbose: bool) -> Path:
     return obj
 
 
+def _build_host(verbose: bool) -> Path:
+    """bd3_host.so: host code only, so g++ and torch's headers and libraries."""
+    from torch.utils import cpp_extension
+    torch_lib = Path(cpp_extension.include_paths()[0]).parent / "lib"
+    rocm = Path(hipcc()).resolve().parent.parent
+    tmp = HOST.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wno-deprecated-declarations",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",  # what torch's HIP headers are compiled with
+           str(CSRC / "host_calls.cpp"), "-o", str(tmp), f"-I{REPO / 'include'}",
+           *(f"-I{p}" for p in cpp_extension.include_paths()), f"-I{rocm / 'include'}",
+           f"-I{sysconfig.get_paths()['include']}", f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu",
+           "-ltorch_hip", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on host_calls.cpp:\n{res.stderr}")
+    os.replace(tmp, HOST)
+    return HOST
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
-    """Compile every .hip source and link libbd3attn.so. Always rebuilds."""
+    """Compile every .hip source, link libbd3attn.so and build bd3_host.so.
+    Always rebuilds."""
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
@@ -80,7 +104,9 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
         raise RuntimeError(f"no .hip sources in {CSRC}")
     jobs = jobs or min(len(sources), os.cpu_count() or 4, 8)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), sources))
+        host.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     res = subprocess.run(cmd, capture_output=True, text=True)

@@ -11,7 +11,7 @@ the same).
 import torch
 from torch import Tensor
 
-from kernels._native import as_kernel_input, check, lib, ptr, stream_of, strides
+from kernels._native import host
 
 
 def _last_stride_1(x: Tensor) -> Tensor:
@@ -39,13 +39,4 @@ def block_sparse_decode_attention(
     """Block-causal attention of the last q_len positions over all kv_len
     keys (reference: kernels/BlockSparseDecodeAttention.py:118-148)."""
     _check_decode_inputs(q, k, v)
-    B, H, q_len, D = q.shape
-    kv_len = k.shape[2]
-    q, k, v = as_kernel_input(_last_stride_1(q)), as_kernel_input(k), as_kernel_input(v)
-    O = torch.empty((B, H, q_len, D), device=q.device, dtype=q.dtype)
-    nbytes = lib().bd3_decode_workspace_bytes(B, H, q_len, kv_len, D, 0)
-    ws = torch.empty(max(nbytes, 1), device=q.device, dtype=torch.uint8)
-    check(lib().bd3_decode(
-        ptr(q), ptr(k), ptr(v), ptr(O), B, H, q_len, kv_len, D, block_size,
-        strides(q, k, v, O), 1.0 / D ** 0.5, ptr(ws), nbytes, stream_of(q)))
-    return O
+    return host().decode(q, k, v, block_size, 0)

@@ -17,7 +17,7 @@ from typing import Any
 import torch
 from torch import Tensor
 
-from kernels._native import as_kernel_input, check, lib, ptr, stream_of, strides
+from kernels._native import host
 
 
 class BlockSparseFlashAttention(torch.autograd.Function):
@@ -45,13 +45,7 @@ class BlockSparseFlashAttention(torch.autograd.Function):
         assert q.dtype == k.dtype == v.dtype == torch.bfloat16, "bf16 inputs only"
         assert D == 64, "head_dim must be 64"
 
-        q, k, v = as_kernel_input(q), as_kernel_input(k), as_kernel_input(v)
-        O = torch.empty((B, H, seq_len, D), device=q.device, dtype=q.dtype)
-        L = torch.empty((B, H, seq_len), device=q.device, dtype=torch.float32)
-        check(lib().bd3_attn_fwd(
-            ptr(q), ptr(k), ptr(v), ptr(O), ptr(L), B, H, n, D, block_size,
-            strides(q, k, v, O), 1.0 / D ** 0.5, stream_of(q)))
-
+        q, k, v, O, L = host().attn_fwd(q, k, v, block_size)
         ctx.save_for_backward(q, k, v, O, L)
         ctx.block_size = block_size
         return O
@@ -60,18 +54,6 @@ class BlockSparseFlashAttention(torch.autograd.Function):
     def backward(ctx: Any, dO: Tensor):  # type: ignore[override]
         q, k, v, O, L = ctx.saved_tensors
         block_size = ctx.block_size
-        B, H, seq_len, D = q.shape
-        n = seq_len // 2
-        assert n % block_size == 0
-
-        dO = as_kernel_input(dO.to(q.dtype))
-        dQ = torch.empty((B, H, seq_len, D), device=q.device, dtype=q.dtype)
-        dK = torch.empty_like(dQ)
-        dV = torch.empty_like(dQ)
-        nbytes = lib().bd3_attn_bwd_workspace_bytes(B, H, n, D)
-        ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-        check(lib().bd3_attn_bwd(
-            ptr(q), ptr(k), ptr(v), ptr(O), ptr(dO), ptr(L), ptr(dQ), ptr(dK), ptr(dV),
-            ptr(ws), nbytes, B, H, n, D, block_size,
-            strides(q, k, v, O, dO, dQ, dK, dV), 1.0 / D ** 0.5, stream_of(q)))
+        assert (q.shape[2] // 2) % block_size == 0
+        dQ, dK, dV = host().attn_bwd(q, k, v, O, L, dO, block_size)
         return dQ, dK, dV, None

@@ -10,10 +10,8 @@ ceil(kv_len / SPLIT_N), :147). Runs bd3_decode_splitkv in libbd3attn.so.
 import torch
 from torch import Tensor
 
-from kernels._native import as_kernel_input, check, lib, ptr, stream_of, strides
-from kernels.BlockSparseDecodeAttention import (
-    _check_decode_inputs, _last_stride_1, block_sparse_decode_attention,
-)
+from kernels._native import host
+from kernels.BlockSparseDecodeAttention import _check_decode_inputs, block_sparse_decode_attention
 
 # keys per split of the reference's default split rule
 SPLIT_N = 256
@@ -38,11 +36,4 @@ def split_kv_decode_attention(
     if n_splits is None:
         n_splits = -(-kv_len // SPLIT_N)
     assert 1 <= n_splits <= kv_len, "n_splits must be in [1, kv_len]"
-    q, k, v = as_kernel_input(_last_stride_1(q)), as_kernel_input(k), as_kernel_input(v)
-    O = torch.empty((B, H, q_len, D), device=q.device, dtype=q.dtype)
-    nbytes = lib().bd3_decode_workspace_bytes(B, H, q_len, kv_len, D, n_splits)
-    ws = torch.empty(max(nbytes, 1), device=q.device, dtype=torch.uint8)
-    check(lib().bd3_decode_splitkv(
-        ptr(q), ptr(k), ptr(v), ptr(O), B, H, q_len, kv_len, D, block_size, n_splits,
-        strides(q, k, v, O), 1.0 / D ** 0.5, ptr(ws), nbytes, stream_of(q)))
-    return O
+    return host().decode(q, k, v, block_size, n_splits)

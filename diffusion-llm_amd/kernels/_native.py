@@ -4,10 +4,15 @@ PyTorch only provides device memory and the current HIP stream here; every
 computation runs in the library's gfx950 kernels. There is no fallback: if
 the library is missing, importing a kernel module still works (so CPU-only
 tooling can inspect signatures) but the first call raises RuntimeError.
+
+The kernel modules make their calls through bd3_host.so (csrc/host_calls.cpp),
+which prepares the tensors and calls the same C ABI natively: `host()`.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from pathlib import Path
@@ -16,6 +21,7 @@ import torch
 
 _PKG = Path(__file__).resolve().parent.parent
 LIB_PATH = Path(os.environ.get("BD3ATTN_LIB", _PKG / "lib" / "libbd3attn.so"))
+HOST_PATH = _PKG / "lib" / "bd3_host.so"
 
 BD3_OK, BD3_EINVAL, BD3_EHIP = 0, 1, 2
 
@@ -94,6 +100,30 @@ def lib() -> ctypes.CDLL:
                     fn.argtypes = args
                 _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """bd3_host.so (see csrc/host_calls.cpp), bound to the loaded library;
+    raise RuntimeError if either was not built."""
+    global _host
+    if _host is None:
+        handle = lib()
+        with _lock:
+            if _host is None:
+                if not HOST_PATH.exists():
+                    raise RuntimeError(
+                        f"{HOST_PATH} not found: build it with "
+                        "`python -c 'import __graft_entry__ as g; g.build()'` "
+                        "(or python diffusion-llm_amd/csrc/build.py)")
+                loader = importlib.machinery.ExtensionFileLoader("bd3_host", str(HOST_PATH))
+                module = importlib.util.module_from_spec(importlib.util.spec_from_loader("bd3_host", loader))
+                loader.exec_module(module)
+                module.bind({n: ctypes.cast(getattr(handle, n), _c_p).value for n in SIGNATURES})
+                _host = module
+    return _host
 
 
 def last_error() -> str:

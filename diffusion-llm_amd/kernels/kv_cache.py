@@ -23,13 +23,12 @@ consumes them immediately, as the reference does).
 """
 from __future__ import annotations
 
-import ctypes
 import math
 
 import torch
 from torch import Tensor
 
-from kernels._native import as_kernel_input, check, lib, ptr, stream_of, strides
+from kernels._native import as_kernel_input, check, host, lib, ptr, stream_of, strides
 
 _MIN_CAPACITY = 256
 
@@ -86,16 +85,20 @@ class KVCache:
         """Make layer_idx's buffers hold `need` tokens of like's
         (batch, heads, *, head_dim) shape and dtype."""
         B, H, _, D = like.shape
+        self._fit(layer_idx, B, H, D, like.dtype, like.device, need)
+
+    def _fit(self, layer_idx: int, B: int, H: int, D: int, dtype: torch.dtype, device: torch.device,
+             need: int) -> None:
         buf = self._k[layer_idx]
         if buf is not None:
-            assert buf.shape[0] == B and buf.shape[1] == H and buf.shape[3] == D, \
-                "cached and new keys differ in batch, heads or head_dim"
-            assert buf.dtype == like.dtype and buf.device == like.device, "cache dtype / device mismatch"
-            if buf.shape[2] >= need:
+            b, h, cap, d = buf.shape
+            assert b == B and h == H and d == D, "cached and new keys differ in batch, heads or head_dim"
+            assert buf.dtype == dtype and buf.device == device, "cache dtype / device mismatch"
+            if cap >= need:
                 return
         cap = max(need, self._capacity or 0, _MIN_CAPACITY, 2 * (buf.shape[2] if buf is not None else 0))
         cap = 8 * math.ceil(cap / 8)
-        k_new = torch.empty((B, H, cap, D), device=like.device, dtype=like.dtype)
+        k_new = torch.empty((B, H, cap, D), device=device, dtype=dtype)
         v_new = torch.empty_like(k_new)
         n = self._len[layer_idx]
         if n > 0:
@@ -150,35 +153,27 @@ def attention_inputs(
     assert W % (3 * n_heads) == 0, "projection width must be 3 * n_heads * head_dim"
     D = W // (3 * n_heads)
     assert D == 64, "head_dim must be 64"
-    if not (qkv.stride(-1) == 1 and qkv.data_ptr() % 16 == 0 and qkv.stride(0) % 8 == 0
-            and qkv.stride(1) % 8 == 0):
-        qkv = qkv.contiguous()
     assert sin_table.dtype == cos_table.dtype == torch.float32 and sin_table.shape == cos_table.shape
     assert sin_table.shape[1] == D // 2, "RoPE tables must be (max_seq_len, head_dim / 2)"
-    sin_table, cos_table = sin_table.contiguous(), cos_table.contiguous()
-    max_pos = sin_table.shape[0]
 
-    pos_ptr, pos0 = None, 0
+    pos0 = 0
     if isinstance(positions, int):
-        pos0 = positions
+        positions, pos0 = None, positions
     elif positions is not None:
         assert positions.shape == (S,), "positions must be (seq,)"
-        positions = positions.to(device=qkv.device, dtype=torch.int64).contiguous()
-        pos_ptr = ptr(positions)
 
-    q = torch.empty((B, n_heads, S, D), device=qkv.device, dtype=qkv.dtype)
-    if kv_cache is None:
-        k_out = torch.empty_like(q)
-        v_out = torch.empty_like(q)
-    else:
-        k_out, v_out = kv_cache.slot(layer_idx, q, S)
-    xstr = (ctypes.c_int64 * 2)(qkv.stride(0), qkv.stride(1))
-    check(lib().bd3_qkv_rope(ptr(qkv), xstr, B, S, n_heads, D, pos_ptr, pos0, ptr(sin_table),
-                             ptr(cos_table), max_pos, ptr(q), ptr(k_out), ptr(v_out),
-                             strides(q, k_out, v_out), stream_of(qkv)))
-    if kv_cache is None:
-        return q, k_out, v_out
-    k_all, v_all = kv_cache.prefix_and_slot(layer_idx, S)
-    if store:
-        kv_cache.commit(layer_idx, S)
+    k_buf = v_buf = None
+    n = 0
+    if type(kv_cache) is KVCache:
+        n = kv_cache._len[layer_idx]
+        kv_cache._fit(layer_idx, B, n_heads, D, qkv.dtype, qkv.device, n + S)
+        k_buf, v_buf = kv_cache._k[layer_idx], kv_cache._v[layer_idx]
+    elif kv_cache is not None:  # a subclass, or another cache with these methods
+        k_buf, v_buf = kv_cache.slot(layer_idx, qkv.new_empty((B, n_heads, S, D)), S)
+    q, k_all, v_all = host().qkv_rope(qkv, n_heads, sin_table, cos_table, positions, pos0, k_buf, v_buf, n)
+    if kv_cache is not None:
+        if type(kv_cache) is not KVCache:
+            k_all, v_all = kv_cache.prefix_and_slot(layer_idx, S)
+        if store:
+            kv_cache.commit(layer_idx, S)
     return q, k_all, v_all

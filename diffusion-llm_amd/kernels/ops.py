@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from kernels._native import as_kernel_input, check, lib, ptr, stream_of, strides
+from kernels._native import host
 
 D = 64
 
@@ -36,13 +36,7 @@ def attn_fwd(q: Tensor, k: Tensor, v: Tensor, block_size: int) -> tuple[Tensor, 
     """BD3-LM training attention forward: O and the natural-log L per row
     (kernels/BlockSparseFlashAttention.py:465-506)."""
     _check_train(q, k, v)
-    B, H, S, _ = q.shape
-    q, k, v = as_kernel_input(q), as_kernel_input(k), as_kernel_input(v)
-    o = q.new_empty((B, H, S, D))
-    lse = q.new_empty((B, H, S), dtype=torch.float32)
-    check(lib().bd3_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(o), ptr(lse), B, H, S // 2, D, block_size,
-                             strides(q, k, v, o), 1.0 / D ** 0.5, stream_of(q)))
-    return o, lse
+    return host().attn_fwd(q, k, v, block_size)[3:]
 
 
 @attn_fwd.register_fake
@@ -55,19 +49,8 @@ def _attn_fwd_fake(q, k, v, block_size):
 def attn_bwd(q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor, dout: Tensor,
              block_size: int) -> tuple[Tensor, Tensor, Tensor]:
     """dQ, dK, dV (kernels/BlockSparseFlashAttention.py:508-562)."""
-    B, H, S, _ = q.shape
-    n = S // 2
-    assert n % block_size == 0, "n must be a multiple of block_size"
-    q, k, v, o = (as_kernel_input(t) for t in (q, k, v, o))
-    dout = as_kernel_input(dout.to(q.dtype))
-    lse = lse.contiguous()
-    dq, dk, dv = (q.new_empty((B, H, S, D)) for _ in range(3))
-    nbytes = lib().bd3_attn_bwd_workspace_bytes(B, H, n, D)
-    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-    check(lib().bd3_attn_bwd(ptr(q), ptr(k), ptr(v), ptr(o), ptr(dout), ptr(lse), ptr(dq), ptr(dk), ptr(dv),
-                             ptr(ws), nbytes, B, H, n, D, block_size, strides(q, k, v, o, dout, dq, dk, dv),
-                             1.0 / D ** 0.5, stream_of(q)))
-    return dq, dk, dv
+    assert (q.shape[2] // 2) % block_size == 0, "n must be a multiple of block_size"
+    return host().attn_bwd(q, k, v, o, lse, dout, block_size)
 
 
 @attn_bwd.register_fake

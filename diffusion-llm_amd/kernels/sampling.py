@@ -22,7 +22,7 @@ import threading
 import torch
 from torch import Tensor
 
-from kernels._native import check, lib, ptr, stream_of
+from kernels._native import host
 
 
 class PhiloxStream:
@@ -64,23 +64,10 @@ def subs_sample_step(
         "logits must be bf16 or fp32 CUDA tensors"
     assert logits.shape[:-1] == block.shape, "block must match the logits' leading dims"
     assert 0.0 <= keep <= 1.0, "keep = s / t must lie in [0, 1]"
-    vocab = logits.shape[-1]
-    rows = block.numel()
-    lg = logits.reshape(rows, vocab)
-    if lg.stride(-1) != 1:
-        lg = lg.contiguous()
-    xt = block.reshape(rows).to(device=logits.device, dtype=torch.int64).contiguous()
-    out = torch.empty_like(xt)
     if u is not None:
         assert u.shape == logits.shape and u.dtype == torch.float64 and u.device == logits.device
-        u = u.reshape(rows, vocab).contiguous()
         seed = offset = 0
     else:
         gen = generator or default_stream()
         seed, offset = gen.seed, gen.next_offset()
-    nbytes = lib().bd3_subs_sample_workspace_bytes(rows, vocab)
-    ws = torch.empty(nbytes, device=lg.device, dtype=torch.uint8) if nbytes else None
-    check(lib().bd3_subs_sample_ws(ptr(lg), lg.stride(0), 1 if lg.dtype == torch.float32 else 0, ptr(xt),
-                                   ptr(out), rows, vocab, mask_index, float(keep), ptr(u), seed, offset,
-                                   ptr(ws), nbytes, stream_of(lg)))
-    return out.view(block.shape)
+    return host().subs_sample(logits, block, mask_index, keep, u, seed, offset)
