@@ -199,22 +199,12 @@ int32_t prefill_auto_splits(int32_t batch, int32_t heads, int32_t q_len, int32_t
 
 int32_t auto_splits(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len) {
   if (q_len >= kPrefillMinQ) return prefill_auto_splits(batch, heads, q_len, kv_len);
-  // A cached step (q_len <= 16, 16-row tiles): at least one workgroup per CU
-  // on a 256-CU part; beyond that more splits only add partial traffic and a
-  // merge launch. Measured at configs[3] (384 workgroups at one split): 66 us
-  // at one split, 68 us at two (including the merge), 71 us at three. Its
-  // merge of up to 32 splits is one memory round trip, so it pays for splits
-  // down to 128 keys, up to 16 of them: 16 queries over a 3584-token cache,
-  // batch 1, 12 heads: 12.7 us at 7 splits, 11.8 at 14 or 16, 12.5-12.9 at
-  // 21-28; over 8192 tokens 16.2 / 13.9 / 15.3 / 15.2 us at 8 / 16 / 22 /
-  // 32; batch 2, 12 heads, over 1024 tokens 11.6 / 11.1 / 10.5 / 11.0 us at
-  // 2 / 4 / 8 / 11.
-  // 32-row tiles (16 < q_len <= 64), whose workgroups take 8 waves when there
-  // are fewer than 256 of them: about 128 workgroups, and at least 1024 keys
-  // per split once there are 64 or more tiles (512 with fewer; the merge
-  // launch costs more than a shorter chain saves): at 8 x 12 heads, q_len 32,
-  // 2048 keys 16.8 us at 2 splits vs 17.8 at 1 and 19.3 at 3; 1024 keys 12.0
-  // at 1 vs 13.7 at 2; batch 1 over 3584 keys 13.3-13.6 at 7-8 splits.
+  // The most ranges a decode call (q_len <= 64) cuts its keys into, which sizes
+  // its workspace; decode_ranges() below takes fewer where that is faster. A
+  // cached step (q_len <= 16): one workgroup per CU, down to 128 keys, at most 16
+  // (its merge of up to 32 is one memory round trip). 32-row tiles: about 128
+  // workgroups, at least 1024 keys a split once there are 64 tiles (512 with
+  // fewer).
   const int64_t base = (int64_t)batch * heads * decode_q_tiles(q_len);
   const int64_t target = q_len <= 16 ? 256 : 128;
   int64_t s = (target + base - 1) / base;
@@ -226,9 +216,25 @@ int32_t auto_splits(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len)
   return (int32_t)s;
 }
 
+// Key ranges a decode call of q_len <= 64 really takes, at most n_splits. More
+// than leave each workgroup a CU of its own (256) only add partials and their
+// merge; and where the library chooses (automatic), splitting must take enough
+// keys off a workgroup's chain (~4.2 us per 1000) to pay for the partials and
+// the merge launch (~4 us). us at 1 split against the count chosen, 12 heads:
+// q_len 16, 1 sequence x 1000 keys 6.8 (6 splits 7.4), x 2000 11.5 / 15: 7.4, x 8192
+// 37.9 / 16: 10.0; 2 x 600 5.8 (4: 7.5); 4 x 3000 17.2 / 5: 11.5; 8 x 1040 8.5 (3: 9.6), x
+// 2064 13.9 / 2: 12.4 (3: 14.1); 16 x 1500 13.6 (2: 16.7), x 4000 30.4 (2: 34.8). q_len 32:
+// 8 x 1056 9.0 (2: 10.3), x 4096 24.7 / 2: 20.9. Asked for: 8 x 1040, q_len 16, 5 splits
+// as 5: 10.4, as 2: 9.0; 8 x 1500, q_len 32, 6 as 6: 16, as 2: 11.9.
+int32_t decode_ranges(int64_t units, int32_t kv_len, int32_t n_splits, bool automatic) {
+  constexpr int64_t kWorkgroups = 256;
+  const int32_t s = (int32_t)std::max<int64_t>(1, std::min<int64_t>(n_splits, kWorkgroups / units));
+  return automatic && kv_len - kv_len / s < 1000 ? 1 : s;
+}
+
 int run_decode(const void* q, const void* k, const void* v, void* o, int32_t batch,
                int32_t heads, int32_t q_len, int32_t kv_len, int32_t block_size,
-               int32_t n_splits, const int64_t* strides, float scale, void* workspace,
+               int32_t n_splits, bool automatic, const int64_t* strides, float scale, void* workspace,
                size_t workspace_bytes, void* stream) {
   if (int st = check_scale(scale)) return st;
   const int q_tiles = decode_q_tiles(q_len);
@@ -237,6 +243,8 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
     return fail(BD3_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
   if (need > 0 && (workspace == nullptr || !aligned16(workspace)))
     return fail(BD3_EINVAL, "workspace must be a 16-byte aligned device pointer");
+  if (q_len < kPrefillMinQ)
+    n_splits = decode_ranges((int64_t)batch * heads * q_tiles, kv_len, n_splits, automatic);
   bd3::DecodeArgs a;
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
@@ -263,22 +271,6 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
   sl = (sl + 31) / 32 * 32;
   a.split_len = sl;
   a.q_tiles = q_tiles;
-  // One workgroup per split, unless that overfills the GPU: then (cached
-  // steps, q_len <= 16) a workgroup computes several consecutive splits and
-  // merges their partials on chip, so that only enough workgroups for one
-  // per CU remain (at configs[3], 384 heads: every split count gives one
-  // workgroup per head, no partials in memory, no merge pass).
-  a.groups = n_splits;
-  a.splits_per_group = 1;
-  const int64_t units = (int64_t)batch * heads * q_tiles;
-  if (q_len <= 16 && n_splits >= 4 && units * n_splits > 512) {
-    const int64_t g = (256 + units - 1) / units;
-    const int per = (int)((n_splits + g - 1) / g);
-    if (per >= 4) {
-      a.splits_per_group = per;
-      a.groups = (n_splits + per - 1) / per;
-    }
-  }
   a.scale_log2 = scale * bd3::kLog2e;
   if (q_len >= kPrefillMinQ) {
     // 128-row tiles, splits of whole 64-key tiles; partials in the same
@@ -289,8 +281,6 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
     }
     int pl = (kv_len + n_splits - 1) / n_splits;
     a.split_len = (pl + 63) / 64 * 64;
-    a.groups = n_splits;
-    a.splits_per_group = 1;
     return hip_status(bd3::launch_prefill(a, static_cast<hipStream_t>(stream)), "prefill launch");
   }
   return hip_status(bd3::launch_decode(a, kDecodeQT, static_cast<hipStream_t>(stream)), "decode launch");
@@ -563,7 +553,7 @@ int bd3_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
   int st = check_common_decode(q, k, v, o, batch, heads, q_len, kv_len, head_dim, block_size, strides);
   if (st) return st;
   const int32_t ns = auto_splits(batch, heads, q_len, kv_len);
-  return run_decode(q, k, v, o, batch, heads, q_len, kv_len, block_size, ns, strides, scale,
+  return run_decode(q, k, v, o, batch, heads, q_len, kv_len, block_size, ns, true, strides, scale,
                     workspace, workspace_bytes, stream);
 }
 
@@ -575,7 +565,7 @@ int bd3_decode_splitkv(const void* q, const void* k, const void* v, void* o, int
   if (st) return st;
   if (n_splits < 1 || n_splits > kv_len)
     return fail(BD3_EINVAL, "n_splits must be in [1, kv_len], got %d", n_splits);
-  return run_decode(q, k, v, o, batch, heads, q_len, kv_len, block_size, n_splits, strides, scale,
+  return run_decode(q, k, v, o, batch, heads, q_len, kv_len, block_size, n_splits, false, strides, scale,
                     workspace, workspace_bytes, stream);
 }
 

@@ -7,10 +7,12 @@
 //
 // decode_partial: one workgroup per (split, 32-row query tile, batch*head).
 //   The split's key range is cut into 32-key chunks that the waves (four, or
-//   eight when the grid has fewer workgroups than CUs and a split holds at
-//   least 16 chunks) take in turn; each wave runs an online softmax over its
-//   chunks, then the waves' states are merged through LDS. With one split the workgroup writes O
-//   directly; otherwise it writes a normalised fp32 partial and its log2-LSE.
+//   eight when the grid leaves a workgroup alone on its CU and a split holds at
+//   least 8 chunks) take in turn; each wave runs an online softmax over its
+//   chunks, then the waves' states are merged through LDS (16 threads per row,
+//   16-byte reads and one 8-byte store each). With one split the workgroup
+//   writes O directly; otherwise it writes a normalised fp32 partial and its
+//   log2-LSE.
 //   K and V are read once per call, with non-temporal loads (ld16_stream) so
 //   the stream does not evict other data from L2 / MALL; measured 7% faster
 //   than cached loads at the configs[3] shape. Each load instruction fetches
@@ -25,13 +27,13 @@
 //   lane is spent on absent queries. Waves step over 32-key chunks fetched
 //   with full-row loads into registers, staged through wave-private LDS
 //   tiles; the loads of a wave's next chunk are in flight while the current
-//   one is computed. When one workgroup per split would overfill the GPU, a
-//   workgroup takes several consecutive splits (splits_per_group): its waves
-//   deal the chunks of all of them out continuously and merge each split's
-//   share into their running state at the split's end (the same LSE merge
-//   the combine pass applies), so the result equals one partial per split
-//   merged, with fewer partials in memory (none when one workgroup covers
-//   all of a head's splits).
+//   one is computed.
+// A call of few workgroups is bound by what each CU can fetch (~55 GB/s from
+// beyond its L2, whatever is in flight: two to four chunks ahead per wave only
+// added their tail reads, 10.0 -> 11.8-14.3 us at 8 x 12 heads, q_len 32, 1056
+// keys) plus ~5 us of launch, first loads and merge; a full one by HBM. The merge
+// in 16-byte pieces and a rescale only when a row's maximum grew took 0.9 us off
+// every 32-row call (10.1 -> 9.2 there; 32 sequences x 4128 keys 65.9 -> 64.6 us).
 // decode_combine: merges the splits, weights exp2(lse_s - max lse) (the
 //   reference's split_kv_reduce_kern arithmetic, :109-127), 4 outputs per
 //   thread.
@@ -42,17 +44,20 @@
 namespace bd3 {
 namespace {
 
-constexpr int kNW = 4;
-constexpr int kThreads = kNW * 64;
+constexpr int kThreads = 256;  // of the merge kernel
 
 constexpr int kQT = 32;       // query rows per workgroup
 constexpr int kSub = 32;      // keys per wave step
 constexpr int kStride = 72;   // padded LDS row (bf16)
 constexpr int kVElems = 2 * kSub * kStride;  // a wave's K and V tiles
 
+// The waves' states for the merge. Rows of O padded to 68 floats: a lane writes
+// its registers' runs of 4 consecutive d as one 16-byte store, the readers
+// take 4 d of a row at a time, and 16 lanes of either hit 16 distinct slots.
+constexpr int kMergeRow = kHeadDim + 4;
 template <int NW>
 struct MergeLds {
-  float o[NW][kHeadDim][kQT + 1];  // O^T per wave (unnormalised), padded
+  float o[NW][kQT][kMergeRow];  // unnormalised
   float m[NW][kQT];
   float l[NW][kQT];
 };
@@ -159,15 +164,17 @@ __global__ __launch_bounds__(NW * 64) void decode_partial(DecodeArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = max_xor32(mx);
-    const float m_new = fmaxf(m, mx * a.scale_log2);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = fast_exp2(m - m_use);
-    m = m_new;
-    lsum *= alpha;
-#pragma unroll
-    for (int db = 0; db < 2; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
+    // Rescale only when some row's maximum grew.
+    const float mt = mx * a.scale_log2;
+    if (__ballot(mt > m) != 0) {
+      const float mn = fmaxf(m, mt);
+      const float alpha = (mn == -INFINITY) ? 1.f : fast_exp2(m - mn);
+      m = mn;
+      lsum *= alpha;
+      oacc[0] *= alpha;
+      oacc[1] *= alpha;
+    }
+    const float m_use = (m == -INFINITY) ? 0.f : m;
 
     float p[16];
 #pragma unroll
@@ -196,41 +203,46 @@ __global__ __launch_bounds__(NW * 64) void decode_partial(DecodeArgs a) {
 #pragma unroll
   for (int db = 0; db < 2; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = 32 * db + 8 * (r >> 2) + 4 * g + (r & 3);
-      ml->o[wave][d][l32] = oacc[db][r];
-    }
+    for (int rg = 0; rg < 4; ++rg)
+      *reinterpret_cast<f32x4*>(&ml->o[wave][l32][32 * db + 8 * rg + 4 * g]) =
+          f32x4{oacc[db][4 * rg], oacc[db][4 * rg + 1], oacc[db][4 * rg + 2], oacc[db][4 * rg + 3]};
   if (g == 0) {
     ml->m[wave][l32] = m;
     ml->l[wave][l32] = lsum;
   }
   __syncthreads();
 
-  const int split_out = a.groups > 1;
+  const int split_out = a.n_splits > 1;
   uint16_t* op = a.o + b * a.so.b + h * a.so.h;
-  const int64_t slot = ((int64_t)bh * a.q_tiles + qt) * a.groups + split;
+  const int64_t slot = ((int64_t)bh * a.q_tiles + qt) * a.n_splits + split;
+  // 16 threads per row, 4 consecutive d each; 4 waves take the rows in two passes.
 #pragma unroll
-  for (int j = 0; j < (kQT * kHeadDim) / kThreads; ++j) {
-    const int e = tid + kThreads * j;
-    const int row = e >> 6, d = e & 63;
-    float mm = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kNW; ++w) mm = fmaxf(mm, ml->m[w][row]);
-    const float mu = (mm == -INFINITY) ? 0.f : mm;
-    float lt = 0.f, ot = 0.f;
+  for (int r0 = 0; r0 < kQT; r0 += kThreads / 16) {
+    const int row = r0 + (tid >> 4), d = 4 * (tid & 15);
+    float mw[kNW], mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kNW; ++w) {
-      const float wgt = fast_exp2(ml->m[w][row] - mu);
+      mw[w] = ml->m[w][row];
+      mm = fmaxf(mm, mw[w]);
+    }
+    const float mu = (mm == -INFINITY) ? 0.f : mm;
+    float lt = 0.f;
+    f32x4 ot = {};
+#pragma unroll
+    for (int w = 0; w < kNW; ++w) {
+      const float wgt = fast_exp2(mw[w] - mu);
       lt += wgt * ml->l[w][row];
-      ot += wgt * ml->o[w][d][row];
+      ot += wgt * *reinterpret_cast<const f32x4*>(&ml->o[w][row][d]);
     }
     if (!split_out) {
       if (i0 + row < a.q_len) {
-        const __bf16 y = (__bf16)(ot / lt);
-        op[(int64_t)(i0 + row) * a.so.s + d] = __builtin_bit_cast(uint16_t, y);
+        const float inv = 1.f / lt;
+        *reinterpret_cast<bf16x4*>(op + (int64_t)(i0 + row) * a.so.s + d) =
+            to_bf16x4(ot[0] * inv, ot[1] * inv, ot[2] * inv, ot[3] * inv);
       }
     } else {
-      a.part_o[(slot * kQT + row) * kHeadDim + d] = lt > 0.f ? ot / lt : 0.f;
+      const float inv = lt > 0.f ? 1.f / lt : 0.f;
+      *reinterpret_cast<f32x4*>(&a.part_o[(slot * kQT + row) * kHeadDim + d]) = ot * inv;
       if (d == 0) a.part_lse[slot * kQT + row] = lt > 0.f ? mm + fast_log2(lt) : -INFINITY;
     }
   }
@@ -259,7 +271,7 @@ constexpr int kLoads16 = kChunk16 * 128 / (64 * 16);  // 16-byte loads per lane 
 
 template <int NW>
 struct Merge16 {
-  float o[NW][kHeadDim][kQ16 + 1];
+  float o[NW][kQ16][kMergeRow];
   float m[NW][kQ16];
   float l[NW][kQ16];
 };
@@ -268,15 +280,12 @@ constexpr size_t smem16_bytes() {
   return sizeof(__bf16) * NW * 2 * kTile16 > sizeof(Merge16<NW>) ? sizeof(__bf16) * NW * 2 * kTile16
                                                                  : sizeof(Merge16<NW>);
 }
-constexpr float kRescale16 = 8.0f;
-
 #ifndef BD3_DEC16_OCC
 #define BD3_DEC16_OCC 4
 #endif
 
 template <int NW>
-__global__ __launch_bounds__(NW * 64, BD3_DEC16_OCC) void decode16_partial(DecodeArgs a) {
-  constexpr int kNT = NW * 64;
+__global__ __launch_bounds__(NW * 64, NW == 4 ? BD3_DEC16_OCC : 2) void decode16_partial(DecodeArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[smem16_bytes<NW>()];
   const int tid = wi_x();
   const int lane = tid & 63;
@@ -286,7 +295,7 @@ __global__ __launch_bounds__(NW * 64, BD3_DEC16_OCC) void decode16_partial(Decod
   __bf16* ks = reinterpret_cast<__bf16*>(smem) + wave * 2 * kTile16;
   __bf16* vs = ks + kTile16;
 
-  const int grp = wg_x();
+  const int split = wg_x();
   const int bh = wg_z();
   const int b = bh / a.heads, h = bh - b * a.heads;
   const uint16_t* qp = a.q + b * a.sq.b + h * a.sq.h;
@@ -349,7 +358,7 @@ __global__ __launch_bounds__(NW * 64, BD3_DEC16_OCC) void decode16_partial(Decod
     mx = fmaxf(mx, shfl_xor(mx, 16));
     mx = max_xor32(mx);
     const float mt = mx * a.scale_log2;
-    if (__ballot(mt > m + kRescale16) != 0) {
+    if (__ballot(mt > m) != 0) {
       const float mn = fmaxf(m, mt);
       const float alpha = (mn == -INFINITY) ? 1.f : fast_exp2(m - mn);
       m = mn;
@@ -384,110 +393,25 @@ __global__ __launch_bounds__(NW * 64, BD3_DEC16_OCC) void decode16_partial(Decod
       *reinterpret_cast<u32x4*>(&vs[off]) = vr[j];
     }
   };
-  // Chunk i of a split's walk is chunk (i + r0) mod n_chunks of the split
-  // (r0 = 7 bh mod n_chunks, the same for every wave). Without that rotation
-  // every workgroup reads the same offset of its head's K/V at the same
-  // time, and the head stride (kv_len x 128 bytes) piles those reads onto
-  // few HBM channels; starting head bh at chunk 7 bh spreads them (measured
-  // 71 -> 66 us at 32 x 12 heads, kv_len 4112, one split).
-  auto split_lo = [&](int sp) { return wave_uniform(sp * a.split_len); };
-  auto split_hi = [&](int sp) { return wave_uniform(imin(sp * a.split_len + a.split_len, key_end)); };
-  auto n_chunks_of = [&](int sp) {
-    const int lo = split_lo(sp), hi = split_hi(sp);
-    return hi > lo ? (hi - lo + kChunk16 - 1) / kChunk16 : 0;
-  };
-  int crot = bh * 7;  // start rotation of the chunks inside a split (mod its chunk count)
-  auto chunk_c0 = [&](int sp, int nc, int i) {
-    const int c = i + (nc > 0 ? crot % nc : 0);
-    return split_lo(sp) + (c >= nc ? c - nc : c) * kChunk16;
-  };
-
-  // The wave's state for the workgroup merge: weights 2^(m - max m), sums l,
-  // unnormalised O (lane shares of l, summed below).
+  // Chunk i of the split's walk is chunk (i + r0) mod n_chunks (r0 = 7 bh mod
+  // n_chunks, the same for every wave). Without that rotation every workgroup
+  // reads the same offset of its head's K/V at the same time, and the head
+  // stride (kv_len x 128 bytes) piles those reads onto few HBM channels;
+  // starting head bh at chunk 7 bh spreads them (measured 71 -> 66 us at 32 x 12
+  // heads, kv_len 4112, one split). The waves take the chunks in turn; each
+  // wave's next chunk streams in while the current one is computed.
   f32x4 o[4] = {};
   float m = -INFINITY, lsum = 0.f;
-  const int s0 = wave_uniform(grp * a.splits_per_group);
-  const int s1 = wave_uniform(imin(s0 + a.splits_per_group, a.n_splits));
-  if (a.splits_per_group == 1) {
-    // One split per workgroup: the waves take its chunks in turn; each
-    // wave's next chunk streams in while the current one is computed.
-    const int hi = split_hi(s0);
-    const int nc = n_chunks_of(s0);
-    if (wave < nc) load(chunk_c0(s0, nc, wave));
-    for (int ch = wave; ch < nc; ch += NW) {
-      stage();
-      if (ch + NW < nc) load(chunk_c0(s0, nc, ch + NW));
-      chunk(chunk_c0(s0, nc, ch), hi, m, lsum, o);
-    }
-  } else {
-    // Several splits per workgroup, computed one after another; the waves
-    // take the chunks in turn (the one-split read pattern). A
-    // wave's share of a split gives a normalised partial and its log2-LSE
-    // (the reference's per-split result, kernels/SplitKVDecodeAttention.py:
-    // 81-87, over the wave's keys of the split), merged into the wave's
-    // running state with the reference's LSE weights (:109-127); the
-    // workgroup merge below combines the waves the same way. The lane shares
-    // of l stay unreduced: m and O are per row, the weights apply to every
-    // share. The next chunk's loads (at a split's end, the wave's first
-    // chunk of the next split) stream in while the current chunk is computed.
-    // The workgroup's chunks, split after split, are dealt to the waves in
-    // turn (chunk g of the sequence to wave g mod NW), so every wave gets the
-    // same count to within one whatever the chunks per split. The head
-    // starts where the one-split order starts it, chunk 7 bh of its chunks
-    // (mod their count): the splits are visited from the one holding that
-    // chunk on (j-th visited: s0 + (j + rot) mod cnt) and each split's chunks
-    // from the same offset on, so heads read different parts of their caches
-    // at any moment (the merge is order-independent up to rounding).
-    const int cnt = s1 - s0;
-    const int ncf = wave_uniform(imax(a.split_len / kChunk16, 1));  // chunks of a full split
-    const int start = wave_uniform((bh * 7) % (cnt * ncf));
-    const int rot = wave_uniform(start / ncf);
-    crot = start - rot * ncf;
-    auto act = [&](int j) { return s0 + (j + rot >= cnt ? j + rot - cnt : j + rot); };
-    int vs = 0, nc = n_chunks_of(act(0)), i = wave;
-    while (vs < cnt && i >= nc) {
-      i -= nc;
-      ++vs;
-      nc = vs < cnt ? n_chunks_of(act(vs)) : 0;
-    }
-    if (vs < cnt) load(chunk_c0(act(vs), nc, i));
-    float ms = -INFINITY, ls = 0.f;
-    f32x4 os[4] = {};
-    while (vs < cnt) {
-      stage();
-      int vs_n = vs, nc_n = nc, i_n = i + NW;
-      while (vs_n < cnt && i_n >= nc_n) {
-        i_n -= nc_n;
-        ++vs_n;
-        nc_n = vs_n < cnt ? n_chunks_of(act(vs_n)) : 0;
-      }
-      if (vs_n < cnt) load(chunk_c0(act(vs_n), nc_n, i_n));
-      const int sp = act(vs);
-      chunk(chunk_c0(sp, nc, i), split_hi(sp), ms, ls, os);
-      if (vs_n != vs) {
-        // the wave's share of split sp is done: merge its normalised partial
-        float lrow = ls + shfl_xor(ls, 16);
-        lrow = sum_xor32(lrow);
-        if (lrow > 0.f) {
-          const float lse = ms + fast_log2(lrow);  // log2-LSE of the share
-          const float mn = fmaxf(m, lse);
-          const float w_old = m == -INFINITY ? 0.f : fast_exp2(m - mn);
-          const float w_new = fast_exp2(lse - mn) / lrow;  // weight of the normalised partial
-          m = mn;
-          // running state: each of the row's 4 lane shares holds a quarter of l
-          lsum = lsum * w_old + 0.25f * fast_exp2(lse - mn);
-#pragma unroll
-          for (int db = 0; db < 4; ++db) o[db] = o[db] * w_old + os[db] * w_new;
-        }
-        ms = -INFINITY;
-        ls = 0.f;
-#pragma unroll
-        for (int db = 0; db < 4; ++db) os[db] = f32x4{};
-      }
-      vs = vs_n;
-      nc = nc_n;
-      i = i_n;
-    }
+  const int lo = wave_uniform(split * a.split_len);
+  const int hi = wave_uniform(imin(lo + a.split_len, key_end));
+  const int nc = hi > lo ? (hi - lo + kChunk16 - 1) / kChunk16 : 0;
+  const int r0 = nc > 0 ? (bh * 7) % nc : 0;
+  auto chunk_c0 = [&](int i) { return lo + (i + r0 >= nc ? i + r0 - nc : i + r0) * kChunk16; };
+  if (wave < nc) load(chunk_c0(wave));
+  for (int ch = wave; ch < nc; ch += NW) {
+    stage();
+    if (ch + NW < nc) load(chunk_c0(ch + NW));
+    chunk(chunk_c0(ch), hi, m, lsum, o);
   }
 
   // Merge the waves' states.
@@ -496,53 +420,42 @@ __global__ __launch_bounds__(NW * 64, BD3_DEC16_OCC) void decode16_partial(Decod
   __syncthreads();  // the K/V tiles are reused below
   Merge16<NW>* ml = reinterpret_cast<Merge16<NW>*>(smem);
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ml->o[wave][16 * db + 4 * hq + r][l16] = o[db][r];
+  for (int db = 0; db < 4; ++db) *reinterpret_cast<f32x4*>(&ml->o[wave][l16][16 * db + 4 * hq]) = o[db];
   if (hq == 0) {
     ml->m[wave][l16] = m;
     ml->l[wave][l16] = lsum;
   }
   __syncthreads();
 
-  // kNT threads x kOut outputs = 16 rows x 64 d.
-  constexpr int kOut = kQ16 * kHeadDim / kNT;
-  constexpr int kTPR = kHeadDim / kOut;  // threads per row
-  const int row = tid / kTPR, d0 = kOut * (tid % kTPR);
-  float mm = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) mm = fmaxf(mm, ml->m[w][row]);
-  const float mu = (mm == -INFINITY) ? 0.f : mm;
-  float lt = 0.f;
-  float ot[kOut] = {};
+  // 256 threads x 4 outputs = 16 rows x 64 d.
+  if (tid >= 256) return;
+  const int row = tid >> 4, d0 = 4 * (tid & 15);
+  float mw[NW], mm = -INFINITY;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    const float wgt = fast_exp2(ml->m[w][row] - mu);
-    lt += wgt * ml->l[w][row];
-#pragma unroll
-    for (int j = 0; j < kOut; ++j) ot[j] += wgt * ml->o[w][d0 + j][row];
+    mw[w] = ml->m[w][row];
+    mm = fmaxf(mm, mw[w]);
   }
-  if (a.groups == 1) {
+  const float mu = (mm == -INFINITY) ? 0.f : mm;
+  float lt = 0.f;
+  f32x4 ot = {};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const float wgt = fast_exp2(mw[w] - mu);
+    lt += wgt * ml->l[w][row];
+    ot += wgt * *reinterpret_cast<const f32x4*>(&ml->o[w][row][d0]);
+  }
+  if (a.n_splits == 1) {
     if (row < a.q_len) {
       const float inv = 1.f / lt;
-      uint16_t* dst = a.o + b * a.so.b + h * a.so.h + (int64_t)row * a.so.s + d0;
-      if constexpr (kOut == 2) {
-        const bf16x4 y = to_bf16x4(ot[0] * inv, ot[1] * inv, 0.f, 0.f);
-        *reinterpret_cast<bf16x2*>(dst) = bf16x2{y[0], y[1]};
-      } else {
-#pragma unroll
-        for (int j = 0; j < kOut; j += 4)
-          *reinterpret_cast<bf16x4*>(dst + j) =
-              to_bf16x4(ot[j] * inv, ot[j + 1] * inv, ot[j + 2] * inv, ot[j + 3] * inv);
-      }
+      *reinterpret_cast<bf16x4*>(a.o + b * a.so.b + h * a.so.h + (int64_t)row * a.so.s + d0) =
+          to_bf16x4(ot[0] * inv, ot[1] * inv, ot[2] * inv, ot[3] * inv);
     }
   } else {
-    const int64_t slot = (int64_t)bh * a.q_tiles * a.groups + grp;  // q_tiles == 1
+    const int64_t slot = (int64_t)bh * a.n_splits + split;  // one query tile
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
-    float* dst = &a.part_o[(slot * kQT + row) * kHeadDim + d0];
-#pragma unroll
-    for (int j = 0; j < kOut; ++j) dst[j] = ot[j] * inv;
-    if (tid % kTPR == 0) a.part_lse[slot * kQT + row] = lt > 0.f ? mm + fast_log2(lt) : -INFINITY;
+    *reinterpret_cast<f32x4*>(&a.part_o[(slot * kQT + row) * kHeadDim + d0]) = ot * inv;
+    if (d0 == 0) a.part_lse[slot * kQT + row] = lt > 0.f ? mm + fast_log2(lt) : -INFINITY;
   }
 }
 
@@ -556,7 +469,7 @@ __global__ __launch_bounds__(kThreads) void decode_combine(DecodeArgs a) {
   const int b = bh / a.heads, h = bh - b * a.heads;
   const int i0 = qt * kQT;
   uint16_t* op = a.o + b * a.so.b + h * a.so.h;
-  const int64_t slot0 = ((int64_t)bh * a.q_tiles + qt) * a.groups;
+  const int64_t slot0 = ((int64_t)bh * a.q_tiles + qt) * a.n_splits;
   const int d0 = 4 * (wi_x() & 15);
 #pragma unroll
   for (int pass = 0; pass < kQT / 16; ++pass) {
@@ -567,7 +480,7 @@ __global__ __launch_bounds__(kThreads) void decode_combine(DecodeArgs a) {
     float mm = -INFINITY, wt = 0.f;
     f32x4 acc = {};
     if constexpr (NS > 0) {
-      const int ns = a.groups;  // <= NS
+      const int ns = a.n_splits;  // <= NS
       float l[NS];
       f32x4 po[NS];
 #pragma unroll
@@ -593,7 +506,7 @@ __global__ __launch_bounds__(kThreads) void decode_combine(DecodeArgs a) {
       // issued before the first use); the same weights, summed in split
       // order.
       constexpr int kG = 8;
-      const int ns = a.groups;
+      const int ns = a.n_splits;
       for (int s0 = 0; s0 < ns; s0 += kG) {
         float l[kG];
 #pragma unroll
@@ -644,29 +557,37 @@ __global__ void mask_dump_kernel(uint8_t* out, int mode, int rows, int cols, int
 }  // namespace
 
 hipError_t launch_decode(const DecodeArgs& a, int /*qt*/, hipStream_t stream) {
-  dim3 grid(a.groups, a.q_tiles, a.bh);
-  if (a.q_len <= kQ16)
-    hipLaunchKernelGGL(decode16_partial<kNW>, grid, dim3(kThreads), 0, stream, a);
-  else if ((int64_t)a.bh * a.q_tiles * a.groups < 256 && a.split_len >= 512)
-    // Fewer workgroups than CUs, each with at least 16 chunks: 8 waves share
-    // them (measured at 8 x 12 heads, q_len 32, one split: 2048 keys 20.9 ->
-    // 17.8 us, 1024 keys 13.4 -> 12.0; batch 1 over 3584 keys 30.1 -> 22.3;
-    // with 128 keys per split 4 waves stay faster, 7.1 vs 7.6 us).
-    hipLaunchKernelGGL(decode_partial<8>, grid, dim3(8 * 64), 0, stream, a);
-  else
-    hipLaunchKernelGGL(decode_partial<kNW>, grid, dim3(kThreads), 0, stream, a);
+  const dim3 grid(a.n_splits, a.q_tiles, a.bh);
+  // At most one workgroup per CU, each with at least 8 chunks: 8 waves share
+  // them (the chunks a wave takes one after another halve). One split, 12 heads
+  // a sequence, us with 4 -> 8 waves: q_len 16, 1 x 600 keys 6.6 -> 5.8, 8 x 1040
+  // 10.5 -> 8.5, 16 x 4000 33.3 -> 30.4; q_len 32, 1 x 1000 9.9 -> 7.9, 8 x 2048
+  // 17.3 -> 14.2; 2 x 1000 at 3 splits of 352 keys 8.8 -> 8.3. 16 waves (147 KB of
+  // LDS) took 1.5 us more at every length up to 2048 keys.
+  const bool wide = (int64_t)a.bh * a.q_tiles * a.n_splits <= 256 && a.split_len >= 256;
+  if (a.q_len <= kQ16) {
+    if (wide)
+      hipLaunchKernelGGL(decode16_partial<8>, grid, dim3(8 * 64), 0, stream, a);
+    else
+      hipLaunchKernelGGL(decode16_partial<4>, grid, dim3(4 * 64), 0, stream, a);
+  } else {
+    if (wide)
+      hipLaunchKernelGGL(decode_partial<8>, grid, dim3(8 * 64), 0, stream, a);
+    else
+      hipLaunchKernelGGL(decode_partial<4>, grid, dim3(4 * 64), 0, stream, a);
+  }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.groups == 1) return e;
+  if (e != hipSuccess || a.n_splits == 1) return e;
   const dim3 cgrid(a.q_tiles, a.bh);
-  if (a.groups == 2)
+  if (a.n_splits == 2)
     hipLaunchKernelGGL(decode_combine<2>, cgrid, dim3(kThreads), 0, stream, a);
-  else if (a.groups == 3)
+  else if (a.n_splits == 3)
     hipLaunchKernelGGL(decode_combine<3>, cgrid, dim3(kThreads), 0, stream, a);
-  else if (a.groups == 4)
+  else if (a.n_splits == 4)
     hipLaunchKernelGGL(decode_combine<4>, cgrid, dim3(kThreads), 0, stream, a);
-  else if (a.groups <= 16)
+  else if (a.n_splits <= 16)
     hipLaunchKernelGGL(decode_combine<16>, cgrid, dim3(kThreads), 0, stream, a);
-  else if (a.groups <= 32)
+  else if (a.n_splits <= 32)
     hipLaunchKernelGGL(decode_combine<32>, cgrid, dim3(kThreads), 0, stream, a);
   else
     hipLaunchKernelGGL(decode_combine<0>, cgrid, dim3(kThreads), 0, stream, a);

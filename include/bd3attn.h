@@ -225,8 +225,8 @@ int bd3_decode(const void* q, const void* k, const void* v, void* o,
                void* stream);
 
 /*
- * Number of key splits bd3_decode / bd3_decode_splitkv use for
- * n_splits == 0 (auto). No reference counterpart.
+ * Number of key splits a bd3_decode call is sized for (its workspace; a call
+ * of q_len <= 64 uses fewer where that is faster). No reference counterpart.
  */
 int32_t bd3_decode_auto_splits(int32_t batch, int32_t heads, int32_t q_len,
                                int32_t kv_len);
@@ -247,6 +247,9 @@ size_t bd3_decode_workspace_bytes(int32_t batch, int32_t heads, int32_t q_len,
  * Split-KV decode attention: the keys [0, kv_len) are cut into n_splits
  * contiguous ranges, each producing a normalised fp32 partial O and its
  * LSE, merged with LSE weights (FlashDecoding). Same result as bd3_decode.
+ * For q_len <= 64 the keys are cut into fewer ranges where n_splits would give
+ * more workgroups than there are CUs (the workspace is sized by n_splits all
+ * the same).
  * The reference's default split count is ceil(kv_len / 256)
  * (kernels/SplitKVDecodeAttention.py:147); callers pass it explicitly.
  * strides: 12 int64 = (b, h, s) element strides of q, k, v, o.

@@ -276,3 +276,31 @@ def test_decode_large_logits(cuda, record_error, q_len, kv_len, n_splits):
     ref = decode_attention(q, k, v, bs)
     torch.cuda.synchronize()
     record_error("O max-abs", max_abs(o, ref), OUT_TOL)
+
+
+# Which kernel and how many key ranges a call takes: eight waves a workgroup
+# from 256 keys a range while there are at most 256 workgroups, four
+# otherwise; fewer ranges than asked for once they would exceed 256 workgroups.
+ROUTES = [(1, 256, 16, 225, 16, 1),   # 256 workgroups of 8 chunks: eight waves, one chunk each
+          (1, 256, 5, 224, 5, 1),     # 7 chunks: four waves
+          (1, 257, 16, 300, 16, 1),   # 257 workgroups: four waves
+          (2, 64, 16, 500, 16, 2),    # 256 workgroups in two ranges, the last one short
+          (3, 43, 16, 511, 16, 2),    # 258: one range
+          (2, 48, 16, 1040, 16, 5),   # five asked for, two taken
+          (8, 38, 1, 700, 4, 4),      # 304 heads: one
+          (2, 64, 32, 513, 32, 2),    # 32-row tiles: 256 workgroups, 9 chunks a range
+          (2, 64, 33, 513, 32, 2),    # two row tiles: one range
+          (1, 12, 64, 1999, 64, 8),   # 192 workgroups of 8 chunks, ragged end
+          (1, 12, 17, 130, 8, 20)]    # more ranges than chunks
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,q_len,kv_len,bs,n_splits", ROUTES)
+def test_decode_routes_match_oracle(cuda, record_error, B, H, q_len, kv_len, bs, n_splits):
+    print(f"decode route B={B} H={H} q_len={q_len} kv_len={kv_len} splits={n_splits}", flush=True)
+    q, k, v = decode_inputs(B, H, q_len, kv_len, seed=H + kv_len)
+    dq, dk, dv = (t.to(cuda, torch.bfloat16) for t in (q, k, v))
+    ref = decode_attention(q, k, v, bs)
+    for o in (splitkv_capi(dq, dk, dv, bs, n_splits), block_sparse_decode_attention(dq, dk, dv, bs)):
+        torch.cuda.synchronize()
+        record_error("decode O max-abs", max_abs(o, ref), OUT_TOL)
