@@ -45,6 +45,10 @@
 // log2(e) are applied in fp32 (dQ: one FMA per element; dK/dV: the chain
 // starts from -L / scale and the result is scaled by scale * log2(e) in the
 // exponent's FMA).
+// Few, long items (a.subs = 2, main launch only): two sets of four waves take an
+//   item's tiles in turn, each set through its own ring, and set 0 adds up at the
+//   end (a dK/dV item's chain is 1.3 us a query tile when its workgroup is alone
+//   on the CU): 1 x 12 heads, n 1024 47.0 -> 35.5 us, n 2048 94.5 -> 66.8 us.
 // Both item kinds load their tiles global -> LDS with global_load_lds into
 // three-stage rings of swizzled tiles (bd3_swz.h), two tiles ahead, with one
 // counted vmcnt wait and barrier per tile, in one LDS buffer of the larger
@@ -120,15 +124,20 @@ __device__ __forceinline__ void dkdv_store(const BwdArgs& a, __bf16* tile, int b
 // are its own 128 rows: wave w's keys are seen only by the rows of 32-row
 // block w % 2 of tile w / 2, so each wave computes that one block (exactly
 // what the tile loop accumulates; its other blocks contribute zeros).
-template <bool MASK16, bool DIAG>
-__device__ __forceinline__ void dkdv_item(const BwdArgs& a, __bf16* smem, int bh, int rank) {
+// SUBS = 2: eight waves, two sets of four that take the walk's tiles in turn,
+// each through a ring of its own (smem_all: SUBS * kBwdLdsBytes); both hold the
+// same keys, and set 0 adds set 1's dK and dV to its own at the end.
+template <bool MASK16, bool DIAG, int SUBS>
+__device__ __forceinline__ void dkdv_item(const BwdArgs& a, __bf16* smem_all, int bh, int rank) {
+  static_assert(SUBS == 1 || !DIAG, "two sets walk whole tiles");
   constexpr int kBK = 128;  // keys per workgroup: 4 waves x 32
-  constexpr int kStages = kDkdvStages;
   constexpr int kStageBytes = kDkdvStageBytes;
 
   const int tid = wi_x();
   const int lane = tid & 63;
-  const int wave = wave_uniform(tid >> 6);
+  const int wave = SUBS == 1 ? wave_uniform(tid >> 6) : wave_uniform((tid >> 6) & 3);  // in its set
+  const int sub = SUBS == 1 ? 0 : wave_uniform(tid >> 8);
+  __bf16* smem = smem_all + sub * (kBwdLdsBytes / 2);
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
@@ -177,8 +186,21 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, __bf16* smem, int bh
   // made in order: tile_of(0), tile_of(1), ...).
   TileWalk walk(t0, n_first, t2);
   TilePtr qn(qp, 2 * qstep, t0, n_first, t2), don(dop, 2 * dostep, t0, n_first, t2);
+  // SUBS = 2: the set's tiles are walk indices sub, sub + 2, ...
+  const int n_mine = SUBS == 1 ? n_tiles : (n_tiles - sub + 1) >> 1;
+  int next = sub;
   auto issue = [&](int stage) {
     const uint32_t st = lds0 + (uint32_t)(stage * kStageBytes) + (uint32_t)wave * 2048u;
+    if constexpr (SUBS == 2) {
+      const int t = wave_uniform(tile_of(next));
+      next += 2;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dma16(qp + t * qstep, qoff[j], st + 1024u * j);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dma16(dop + t * dostep, dooff[j], st + 8192u + 1024u * j);
+      if (wave == 0) dma16_va(scal_src + t * kSwRows, lds0 + (uint32_t)(stage * kStageBytes) + 16384u);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) dma16(qn.cur, qoff[j], st + 1024u * j);
 #pragma unroll
@@ -200,8 +222,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, __bf16* smem, int bh
   };
 
   // Tiles 0 and 1 are requested before the K / V rows are waited for.
-  issue(0);
-  if (n_tiles > 1) issue(1);
+  if (SUBS == 1 || n_mine > 0) issue(0);
+  if (n_mine > 1) issue(1);
   // V rows are kept negated: the dP products then start from Delta and give
   // Delta - dP directly (no per-element subtraction), so the kernel forms
   // -dS = P o (Delta - dP) and negates dK once at the end.
@@ -305,15 +327,16 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, __bf16* smem, int bh
     return;
   }
   int cur = 0;
-  for (int it = 0; it < n_tiles; ++it) {
-    const bool pf = it + 2 < n_tiles;
+  const int steps = SUBS == 1 ? n_tiles : (n_tiles + 1) >> 1;  // of the set with more tiles
+  for (int it = 0; it < steps; ++it) {
+    const bool pf = it + 2 < n_mine;
     if (pf) issue(cur == 0 ? 2 : cur - 1);
-    const int q0 = wave_uniform(tile_of(it) * kSwRows);
+    const int q0 = wave_uniform(tile_of(SUBS == 1 ? it : imin(2 * it + sub, n_tiles - 1)) * kSwRows);
     const int c0 = bounds_class(cb, q0, 32, a.n);
     const int c1 = bounds_class(cb, q0 + 32, 32, a.n);
     // One code path for every live tile (the accumulators are updated by one
     // set of instructions, so they keep their registers).
-    if ((c0 | c1) != kNone) {
+    if ((SUBS == 1 || it < n_mine) && (c0 | c1) != kNone) {
       const __bf16* qs = &smem[cur * (kStageBytes / 2)];
       const __bf16* dos = qs + kSwTile;
       const float* scal = reinterpret_cast<const float*>(qs + 2 * kSwTile);
@@ -345,6 +368,32 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, __bf16* smem, int bh
     cur = cur == 2 ? 0 : cur + 1;
   }
 
+  if constexpr (SUBS == 2) {
+    // Through LDS, every wave past its last read of the rings: 16 KB a wave,
+    // then the store's regions behind them.
+    static_assert(4 * 64 * 256 + 4 * kTileElems * 2 <= 2 * kBwdLdsBytes, "hand-over and store regions fit");
+    float* ex = reinterpret_cast<float*>(smem_all) + wave * (64 * 64) + lane;
+    if (sub == 1) {
+#pragma unroll
+      for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          ex[(16 * db + r) * 64] = dk[db][r];
+          ex[(32 + 16 * db + r) * 64] = dv[db][r];
+        }
+    }
+    __syncthreads();
+    if (sub == 1) return;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        dk[db][r] += ex[(16 * db + r) * 64];
+        dv[db][r] += ex[(32 + 16 * db + r) * 64];
+      }
+    dkdv_store(a, smem_all + 4 * 64 * 128 + wave * kTileElems, bo.b, bo.h, kw, lane, dk, dv);
+    return;
+  }
   dkdv_store(a, smem + wave * kTileElems, bo.b, bo.h, kw, lane, dk, dv);
 }
 
@@ -488,11 +537,15 @@ __device__ __forceinline__ void diag_block(const BwdArgs& a, __bf16* smem, int b
 // n/128 - 1 - r/2 of the clean half for even r, of the noisy half for odd r)
 // of (batch*head) bh, with the ring in `smem` (kDqLdsBytes). Delta and the
 // rows' L come from the Delta pass.
-template <bool MASK16>
-__device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem, int bh, int rank) {
+// SUBS = 2: two sets of four waves as in dkdv_item; set 0 also takes the folded
+// diagonal tiles and adds set 1's dQ to its own.
+template <bool MASK16, int SUBS>
+__device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem_all, int bh, int rank) {
   constexpr int kBM = 128;  // query rows per workgroup: 4 waves x 32
   constexpr int kStages = kDqStages;
   constexpr int kAhead = kStages - 1;  // tiles requested ahead of the one being computed
+  const int sub = SUBS == 1 ? 0 : wave_uniform((int)threadIdx.x >> 8);
+  __bf16* smem = smem_all + sub * (kBwdLdsBytes / 2);
   auto stage_k = [&](int st) { return smem + st * (2 * kSwTile); };
   auto stage_v = [&](int st) { return smem + st * (2 * kSwTile) + kSwTile; };
 
@@ -501,7 +554,7 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem, int bh, 
   // configs[1], outputs identical).
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = wave_uniform(tid >> 6);
+  const int wave = SUBS == 1 ? wave_uniform(tid >> 6) : wave_uniform((tid >> 6) & 3);  // in its set
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
@@ -554,8 +607,23 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem, int bh, 
   // Sources of the next tile to request, walked tile by tile.
   TileWalk walk(t0, n_first, t2);
   TilePtr kn(kp, 2 * kstep, t0, n_first, t2), vn(vp, 2 * vstep, t0, n_first, t2);
+  // The loop's tiles; SUBS = 2: the set's j-th tile is walk index sub + 2j, and
+  // set 0's last two are the folded diagonal ones.
+  const int n_loop = fold ? n_tiles - 2 : n_tiles;
+  const int n_mine = SUBS == 1 ? n_loop : (n_loop - sub + 1) >> 1;
+  const int n_loads = SUBS == 1 ? n_tiles : n_mine + (fold && sub == 0 ? 2 : 0);
+  int next = 0;
   auto issue = [&](int stage) {
     const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
+    if constexpr (SUBS == 2) {
+      const int t = wave_uniform(tile_of(next < n_mine ? sub + 2 * next : n_loop + next - n_mine));
+      ++next;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dma16(kp + t * kstep, koff[j], dst + 1024u * j);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) dma16(vp + t * vstep, voff[j], dst + 8192u + 1024u * j);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) dma16(kn.cur, koff[j], dst + 1024u * j);
 #pragma unroll
@@ -569,7 +637,7 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem, int bh, 
   // The first kAhead tiles are requested before the row loads are waited for.
 #pragma unroll
   for (int i = 0; i < kAhead; ++i)
-    if (i < n_tiles) issue(i);
+    if (i < n_loads) issue(i);
   const float lrow = lse_row * kLog2e;
 #pragma unroll
   for (int c = 0; c < 4; ++c) asm volatile("" ::"v"(qreg[c]), "v"(doreg[c]));
@@ -626,17 +694,17 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem, int bh, 
   // the two diagonal tiles (the walk's last) are left to diag_block; a noisy
   // row tile also sees clean keys, so the loop keeps at least one tile.
   vm_wait_barrier<0>();
-  const int n_loop = fold ? n_tiles - 2 : n_tiles;
   int cur = 0;
-  for (int it = 0; it < n_loop; ++it) {
-    const bool pf = it + kAhead < n_tiles;
+  const int steps = SUBS == 1 ? n_loop : (n_loop + 1) >> 1;  // of the set with more tiles
+  for (int it = 0; it < steps; ++it) {
+    const bool pf = it + kAhead < n_loads;
     if (pf) issue(cur + kAhead < kStages ? cur + kAhead : cur + kAhead - kStages);
-    const int k0 = wave_uniform(tile_of(it) * kSwRows);
+    const int k0 = wave_uniform(tile_of(SUBS == 1 ? it : imin(2 * it + sub, n_loop - 1)) * kSwRows);
     const int c0 = bounds_class(cb, k0, 32, a.n);
     const int c1 = bounds_class(cb, k0 + 32, 32, a.n);
     // One code path for every live tile (the accumulators keep their registers):
     // its two 32-key blocks one after the other, each straight into dQ.
-    if ((c0 | c1) != kNone) {
+    if ((SUBS == 1 || it < n_mine) && (c0 | c1) != kNone) {
       const __bf16* ks = stage_k(cur);
       const __bf16* vs = stage_v(cur);
 #pragma unroll
@@ -667,9 +735,30 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, __bf16* smem, int bh, 
     // flight) and no wave still in the loop: waves 0, 1 take their keys from
     // the first diagonal tile, waves 2, 3 from the second.
     vm_wait_barrier<0>();
-    const int sd = (n_tiles - 2 + (wave >> 1)) % kStages;
-    diag_block<MASK16>(a, smem, bo.b, bo.h, qrow0, wave, lane, stage_k(sd), stage_v(sd), qreg, doreg, lse_row, drow,
-                       dq);
+    const int sd = ((SUBS == 1 ? n_tiles - 2 : n_mine) + (wave >> 1)) % kStages;
+    if (SUBS == 1 || sub == 0)
+      diag_block<MASK16>(a, smem, bo.b, bo.h, qrow0, wave, lane, stage_k(sd), stage_v(sd), qreg, doreg, lse_row, drow,
+                         dq);
+    else
+      __syncthreads();  // the one in diag_block
+  }
+  if constexpr (SUBS == 2) {
+    // Through set 1's ring, which none of its waves reads any more.
+    float* ex = reinterpret_cast<float*>(smem_all + kBwdLdsBytes / 2) + wave * (32 * 64) + lane;
+    if (sub == 1) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        ex[r * 64] = dq[0][r];
+        ex[(16 + r) * 64] = dq[1][r];
+      }
+    }
+    __syncthreads();
+    if (sub == 1) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      dq[0][r] += ex[r * 64];
+      dq[1][r] += ex[(16 + r) * 64];
+    }
   }
   uint16_t* dqp = a.dq + bo.b * a.sdq.b + bo.h * a.sdq.h + (int64_t)myq * a.sdq.s;
 #pragma unroll
@@ -729,20 +818,20 @@ __global__ __launch_bounds__(256) void attn_bwd_delta_kernel(BwdArgs a) {
 // pass's planes, so they need no ordering between them, and one launch has
 // one start-up and one tail instead of two. One LDS buffer serves either
 // kind's ring.
-template <int OCC, bool MASK16>
-__global__ __launch_bounds__(256, OCC) void attn_bwd_kernel(BwdArgs a) {
-  __shared__ __attribute__((aligned(1024))) __bf16 smem[kBwdLdsBytes / 2];
+template <int OCC, bool MASK16, int SUBS>
+__global__ __launch_bounds__(256 * SUBS, OCC) void attn_bwd_kernel(BwdArgs a) {
+  __shared__ __attribute__((aligned(1024))) __bf16 smem[SUBS * kBwdLdsBytes / 2];
   const int id = wg_x();
   const int slot = id / a.bh, bh = id - slot * a.bh;
   const int code = a.n_items <= kBwdOrderMax ? (int)a.order[slot] : a.first_code + slot;
   const int dq_items = 2 * a.n / 128;
   const int dk_rank = code - dq_items;
   if (code < dq_items)
-    dq_item<MASK16>(a, smem, bh, code);
-  else if (dk_rank >= a.n / 128 && 32 % a.bs == 0)  // a noisy key tile, blocks within 32 keys
-    dkdv_item<MASK16, true>(a, smem, bh, dk_rank);
+    dq_item<MASK16, SUBS>(a, smem, bh, code);
+  else if (SUBS == 1 && dk_rank >= a.n / 128 && 32 % a.bs == 0)  // a noisy key tile, blocks within 32 keys
+    dkdv_item<MASK16, SUBS == 1, SUBS>(a, smem, bh, dk_rank);
   else
-    dkdv_item<MASK16, false>(a, smem, bh, dk_rank);
+    dkdv_item<MASK16, false, SUBS>(a, smem, bh, dk_rank);
 }
 
 }  // namespace
@@ -759,11 +848,16 @@ hipError_t launch_attn_bwd_items(const BwdArgs& a, hipStream_t stream) {
   // 51 KB of LDS). Measured against two waves per SIMD with the dK/dV
   // items' four product chains interleaved (230 VGPRs): 258 vs 276 us at
   // B=4, H=16, n=2048, 348 vs 380 at B=2, H=12, n=4096, 689 vs 746 at n=8192.
-  const dim3 grid(a.bh * a.n_items), block(256);
-  if (a.bs % 16 == 0)
-    hipLaunchKernelGGL((attn_bwd_kernel<3, true>), grid, block, 0, stream, a);
+  const dim3 grid(a.bh * a.n_items), block(256 * a.subs);
+  if (a.subs == 2) {
+    if (a.bs % 16 == 0)
+      hipLaunchKernelGGL((attn_bwd_kernel<2, true, 2>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((attn_bwd_kernel<2, false, 2>), grid, block, 0, stream, a);
+  } else if (a.bs % 16 == 0)
+    hipLaunchKernelGGL((attn_bwd_kernel<3, true, 1>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((attn_bwd_kernel<3, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attn_bwd_kernel<3, false, 1>), grid, block, 0, stream, a);
   return hipGetLastError();
 }
 

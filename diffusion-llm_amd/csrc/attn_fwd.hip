@@ -35,6 +35,12 @@
 // more than kRescale (log2 units); otherwise the stale max is kept, which
 // bounds P by 2^kRescale and leaves O / l exact.
 //
+// Few, long items (a.subs = 2): a lone workgroup per CU runs one wave per SIMD,
+// and its walk is one chain of load, product, softmax and barrier latencies
+// (~1 us a tile). Two sets of four waves then share the walk, tile by tile in
+// turn, through a ring each, and merge at the end: 1 x 12 heads, n 1024 18.5 ->
+// 15.5 us, n 2048 33.9 -> 28.4 us.
+//
 // Prefill mode (prefill_attn_kernel, DecodeArgs): the same body over the
 // decode mask when many queries attend to the cache at once (the uncached
 // block-causal prefill of kernels/BlockSparseDecodeAttention.py:40-110 with
@@ -72,16 +78,22 @@ constexpr float kRescale = 8.0f;
 // no mask arithmetic. MASK16: every row's key intervals start and end on
 // multiples of 16 (training: the block size is a multiple of 16; prefill:
 // the block size and kv_len are).
-template <bool MASK16, bool PREFILL, class Args>
+// SUBS = 2 (training): eight waves, two sets of four that take the walk's tiles
+// in turn, each through a ring of its own; both hold the same rows, and their
+// (reference, sum, O) are merged at the end.
+template <bool MASK16, bool PREFILL, int SUBS, class Args>
 __device__ __forceinline__ void fwd_body(Args a) {
   constexpr int kBM = 128;  // query rows per workgroup: 4 waves x 32
   constexpr int kStages = BD3_FWD_STAGES;
   constexpr int kAhead = kStages - 1;  // tiles requested ahead of the one being computed
-  __shared__ __attribute__((aligned(1024))) __bf16 smem[kStages][2][kSwTile];  // [stage][K|V]
+  __shared__ __attribute__((aligned(1024))) __bf16 smem_all[SUBS][kStages][2][kSwTile];  // [set][stage][K|V]
+  static_assert(SUBS == 1 || (!PREFILL && kStages == 2), "two sets: training, two-stage rings");
 
   const int tid = wi_x();
   const int lane = tid & 63;
-  const int wave = wave_uniform(tid >> 6);
+  const int wave = SUBS == 1 ? wave_uniform(tid >> 6) : wave_uniform((tid >> 6) & 3);  // in its set
+  const int sub = SUBS == 1 ? 0 : wave_uniform(tid >> 8);
+  auto& smem = smem_all[sub];
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
@@ -157,6 +169,15 @@ __device__ __forceinline__ void fwd_body(Args a) {
   // made in order: tile_of(0), tile_of(1), ...).
   TileWalk walk(t0, n_first, t2);
   TilePtr kn(kp, 2 * kstep, t0, n_first, t2), vn(vp, 2 * vstep, t0, n_first, t2);
+  // SUBS = 2: walk index i into a stage of the set's ring.
+  auto issue_at = [&](int stage, int i) {
+    const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
+    const int t = wave_uniform(tile_of(i));
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(kp + t * kstep, koff[j], dst + 1024u * j);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(vp + t * vstep, voff[j], dst + 8192u + 1024u * j);
+  };
   auto issue = [&](int stage) {
     const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
     uint32_t ko[2] = {koff[0], koff[1]}, vo[2] = {voff[0], voff[1]};
@@ -192,7 +213,19 @@ __device__ __forceinline__ void fwd_body(Args a) {
   // the direct loads issued after them, which is harmless.
   bool diag_first = false;
   if constexpr (!PREFILL && kStages == 2) diag_first = q0 < a.n && 32 % a.bs == 0;
-  if (diag_first) {
+  // SUBS = 2: the set's tiles are walk indices i0, i0 + 2, ...; with the
+  // diagonal step, which set 0 takes, set 1 starts the loop.
+  const int n_diag = diag_first ? 2 : 0;
+  const int i0 = n_diag + (diag_first ? 1 - sub : sub);
+  const int n_mine = imax(0, (n_tiles - i0 + 1) >> 1);
+  if constexpr (SUBS == 2) {
+    if (diag_first && sub == 0) {
+      issue_at(0, 0);
+      issue_at(1, 1);
+    } else if (n_mine > 0) {
+      issue_at(0, i0);
+    }
+  } else if (diag_first) {
     issue(0);
     issue(1);
   } else {
@@ -382,38 +415,90 @@ __device__ __forceinline__ void fwd_body(Args a) {
   // Every row group sees at least its own block, so n_tiles >= 1.
   vm_wait_barrier<0>();
 
-  int it = 0, cur = 0;
-  if (diag_first) {
-    // Wave w's block lies in half w % 2 of tile w / 2 (stage w / 2). Once
-    // every wave holds its operands, stage 0 takes the first tile of the
-    // loop, which loads while the blocks are formed.
-    const int st = wave >> 1;
-    step(std::integral_constant<int, 1>(), std::true_type(), wave & 1, wave_uniform(tile_of(st) * kSwRows),
-         a.bs == 32 ? kFull : kPartial, smem[st][0], smem[st][1], [&] {
-           vm_wait_barrier<0>();
-           if (n_tiles > 2) issue(0);
-         });
-    it = 2;
-    vm_wait_barrier<0>();
-  }
-  for (; it < n_tiles; ++it) {
-    const bool pf = it + kAhead < n_tiles;
-    if (pf) issue(cur + kAhead < kStages ? cur + kAhead : cur + kAhead - kStages);
-    const int k0 = wave_uniform(tile_of(it) * kSwRows);
-    // The tile's class for this wave's rows.
-    if (walk_live(wc, it, n_first))
-      step(std::integral_constant<int, 2>(), std::false_type(), 0, k0,
-           walk_full(wc, it, n_first) ? kFull : kPartial, smem[cur][0], smem[cur][1], [] {});
-    // Tile it+1 complete (the loads of later tiles may stay in flight), and
-    // every wave is done reading stage `cur` before it is refilled.
-    if (pf)
-      vm_wait_barrier<4 * (kAhead - 1)>();
-    else
+  if constexpr (SUBS == 1) {
+    int it = 0, cur = 0;
+    if (diag_first) {
+      // Wave w's block lies in half w % 2 of tile w / 2 (stage w / 2). Once
+      // every wave holds its operands, stage 0 takes the first tile of the
+      // loop, which loads while the blocks are formed.
+      const int st = wave >> 1;
+      step(std::integral_constant<int, 1>(), std::true_type(), wave & 1, wave_uniform(tile_of(st) * kSwRows),
+           a.bs == 32 ? kFull : kPartial, smem[st][0], smem[st][1], [&] {
+             vm_wait_barrier<0>();
+             if (n_tiles > 2) issue(0);
+           });
+      it = 2;
       vm_wait_barrier<0>();
-    cur = cur + 1 == kStages ? 0 : cur + 1;
+    }
+    for (; it < n_tiles; ++it) {
+      const bool pf = it + kAhead < n_tiles;
+      if (pf) issue(cur + kAhead < kStages ? cur + kAhead : cur + kAhead - kStages);
+      const int k0 = wave_uniform(tile_of(it) * kSwRows);
+      // The tile's class for this wave's rows.
+      if (walk_live(wc, it, n_first))
+        step(std::integral_constant<int, 2>(), std::false_type(), 0, k0,
+             walk_full(wc, it, n_first) ? kFull : kPartial, smem[cur][0], smem[cur][1], [] {});
+      // Tile it+1 complete (the loads of later tiles may stay in flight), and
+      // every wave is done reading stage `cur` before it is refilled.
+      if (pf)
+        vm_wait_barrier<4 * (kAhead - 1)>();
+      else
+        vm_wait_barrier<0>();
+      cur = cur + 1 == kStages ? 0 : cur + 1;
+    }
+  } else {
+    if (diag_first) {
+      // As below; set 1 only meets the two barriers.
+      if (sub == 0) {
+        const int st = wave >> 1;
+        step(std::integral_constant<int, 1>(), std::true_type(), wave & 1, wave_uniform(tile_of(st) * kSwRows),
+             a.bs == 32 ? kFull : kPartial, smem[st][0], smem[st][1], [&] {
+               vm_wait_barrier<0>();
+               if (n_mine > 0) issue_at(0, i0);
+             });
+      } else {
+        vm_wait_barrier<0>();
+      }
+      vm_wait_barrier<0>();
+    }
+    const int steps = (n_tiles - n_diag + 1) >> 1;  // of the set with more tiles
+    for (int j = 0; j < steps; ++j) {
+      const int i = i0 + 2 * j, cur = j & 1;
+      if (j + 1 < n_mine) issue_at(cur ^ 1, i + 2);
+      if (j < n_mine && walk_live(wc, i, n_first))
+        step(std::integral_constant<int, 2>(), std::false_type(), 0, wave_uniform(tile_of(i) * kSwRows),
+             walk_full(wc, i, n_first) ? kFull : kPartial, smem[cur][0], smem[cur][1], [] {});
+      vm_wait_barrier<0>();
+    }
   }
 
-  const float ltot = sum_xor32(lsum);
+  float ltot = sum_xor32(lsum);
+  if constexpr (SUBS == 2) {
+    // Set 1 hands its state over through LDS (every wave is past its last read
+    // of the rings); a set that met no key of a row has l = 0.
+    float* ex = reinterpret_cast<float*>(&smem_all[0][0][0][0]) + wave * (34 * 64) + lane;
+    if (sub == 1) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        ex[r * 64] = o[0][r];
+        ex[(16 + r) * 64] = o[1][r];
+      }
+      ex[32 * 64] = mref;
+      ex[33 * 64] = ltot;
+    }
+    __syncthreads();
+    if (sub == 1) return;
+    const float m1 = ex[32 * 64], l1 = ex[33 * 64];
+    const float m = l1 > 0.f ? (ltot > 0.f ? fmaxf(mref, m1) : m1) : mref;
+    const float w0 = ltot > 0.f ? fast_exp2(mref - m) : 0.f, w1 = l1 > 0.f ? fast_exp2(m1 - m) : 0.f;
+    mref = m;
+    ltot = ltot * w0 + l1 * w1;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      o[0][r] = o[0][r] * w0 + ex[r * 64] * w1;
+      o[1][r] = o[1][r] * w0 + ex[(16 + r) * 64] * w1;
+    }
+  }
   if constexpr (PREFILL) {
     if (myq >= a.q_len) return;
     // A row may see no key of a later split: O = 0, LSE = -inf.
@@ -454,14 +539,14 @@ __device__ __forceinline__ void fwd_body(Args a) {
   }
 }
 
-template <int OCC, bool MASK16>
-__global__ __launch_bounds__(256, OCC) void attn_fwd_dma_kernel(FwdArgs a) {
-  fwd_body<MASK16, false>(a);
+template <int OCC, bool MASK16, int SUBS>
+__global__ __launch_bounds__(256 * SUBS, OCC) void attn_fwd_dma_kernel(FwdArgs a) {
+  fwd_body<MASK16, false, SUBS>(a);
 }
 
 template <int OCC, bool MASK16>
 __global__ __launch_bounds__(256, OCC) void prefill_attn_kernel(DecodeArgs a) {
-  fwd_body<MASK16, true>(a);
+  fwd_body<MASK16, true, 1>(a);
 }
 
 // Merges the split partials of the rows whose 128-row tile spans several
@@ -542,12 +627,18 @@ __global__ __launch_bounds__(512) void prefill_combine(DecodeArgs a) {
 
 
 hipError_t launch_attn_fwd(const FwdArgs& a, hipStream_t stream) {
-  // n % 128 == 0 always holds (validated): 128-row query tiles of 4 waves.
-  const dim3 grid(a.bh * (2 * a.n / 128)), block(256);
-  if (a.bs % 16 == 0)
-    hipLaunchKernelGGL((attn_fwd_dma_kernel<BD3_FWD_OCC, true>), grid, block, 0, stream, a);
+  // n % 128 == 0 always holds (validated): 128-row query tiles of 4 waves, or
+  // of two sets of 4 (a.subs).
+  const dim3 grid(a.bh * (2 * a.n / 128)), block(256 * a.subs);
+  if (a.subs == 2) {
+    if (a.bs % 16 == 0)
+      hipLaunchKernelGGL((attn_fwd_dma_kernel<4, true, 2>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((attn_fwd_dma_kernel<4, false, 2>), grid, block, 0, stream, a);
+  } else if (a.bs % 16 == 0)
+    hipLaunchKernelGGL((attn_fwd_dma_kernel<BD3_FWD_OCC, true, 1>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((attn_fwd_dma_kernel<BD3_FWD_OCC, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attn_fwd_dma_kernel<BD3_FWD_OCC, false, 1>), grid, block, 0, stream, a);
   return hipGetLastError();
 }
 

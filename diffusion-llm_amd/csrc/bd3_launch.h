@@ -28,6 +28,7 @@ struct FwdArgs {
   int bh;  // batch * heads
   int n;
   int bs;
+  int subs;  // sets of 4 waves per workgroup, 1 or 2
   float scale_log2;  // softmax scale * log2(e)
 };
 
@@ -53,6 +54,7 @@ struct BwdArgs {
   // diagonal blocks are live) are formed at the end of the dQ items of the
   // same rows, and the launch holds no dK/dV item for them.
   int fold_diag;
+  int subs;  // sets of 4 waves per workgroup, 1 or 2 (both kinds of items in the launch)
   Strides3 sq, sk, sv, so, sdo, sdq, sdk, sdv;
   int heads;
   int bh;

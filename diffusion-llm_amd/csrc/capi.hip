@@ -130,6 +130,44 @@ bd3::BwdArgs bwd_args(const void* q, const void* k, const void* v, const void* o
   return a;
 }
 
+// Sets of four waves per workgroup of the training launches: two where a few
+// long items leave the chip idle (the sets take an item's tiles in turn and add
+// up at its end), one where the launch is bound by its work. Both rules weigh
+// the longest item's chain against the load per workgroup slot; a two-set
+// workgroup's chain is 1.25-1.45 times shorter, but fewer of them fit (backward
+// 256 for 768, forward 512 of twice the waves for 1024) and each start-up is
+// longer. Fitted to 33 shapes, 12 heads a sequence, block 16, us with one -> two:
+// backward main launch 1 x n 256 14.9 -> 13.4, 1 x 1024 47.0 -> 35.5, 1 x 2048 94.5
+// -> 66.8, 1 x 3072 156.6 -> 129.4, 2 x 1024 51.4 -> 42.4, 3 x 512 28.0 -> 24.7; not 4 x
+// 512 32.8 (33.6), 3 x 1024 57.6 (59.1), 2 x 2048 116.5 (121.8), 8 x 256 19.9 (26.2),
+// 8 x 1024 115 (149). Forward 1 x 1024 18.5 -> 15.5, 1 x 2048 33.9 -> 28.4, 2 x 1024
+// 20.2 -> 18.8, 1 x 4096 76.8 -> 72.9; not 8 x 256 10.7 (11.3), 3 x 1024 23.1 (23.0), 6
+// x 512 16.5 (18.3), 8 x 1024 41.6 (47.1).
+
+// longest, total: cost units of the longest item and of all of them (3 a tile for
+// a dQ item, 4 for a dK/dV item); items of all batch*heads. Times in us.
+int bwd_subs(int longest, int64_t total, int64_t items) {
+  const double load = (double)total / 768.0;
+  const double chain1 = 5.0 + 0.33 * longest, work1 = 5.0 + 0.68 * load + 8.1 * (double)items / 768.0;
+  const double chain2 = 6.0 + 0.23 * longest, work2 = 4.0 + 0.85 * load + 4.5 * (double)items / 256.0;
+  // one set: the two overlap only in part
+  const double one = std::cbrt(chain1 * chain1 * chain1 + work1 * work1 * work1);
+  return longest >= 32 && std::max(chain2, work2) < 0.93 * one ? 2 : 1;
+}
+
+int fwd_subs(const bd3::FwdArgs& a) {
+  int longest = 0;
+  int64_t total = 0;
+  for (int q0 = 0; q0 < 2 * a.n; q0 += 128) {
+    const bd3::KeyRanges kr = bd3::train_key_ranges(q0, 128, a.n, a.bs, 64);
+    const int tiles = (kr.t1 - kr.t0) + (kr.t3 - kr.t2);
+    longest = std::max(longest, tiles);
+    total += tiles;
+  }
+  const double load = (double)(total * a.bh) / 1024.0;
+  return longest >= 8 && load < longest * (0.2 + longest / 300.0) ? 2 : 1;
+}
+
 // The backward's work items of one batch*head in launch order, longest
 // first: a stable sort on each item's MFMA work, the tiles it walks times
 // the products per tile (a dQ query tile three: S, dP, dQ; a dK/dV key tile
@@ -141,6 +179,7 @@ void bwd_order(bd3::BwdArgs& a, bool dq, bool dkdv) {
   // key tiles' diagonal blocks are formed by the dQ items of the same rows
   // (see attn_bwd.hip), so the dK/dV items are the clean key tiles only.
   a.fold_diag = dq && dkdv && 32 % a.bs == 0;
+  a.subs = 1;
   a.first_code = dq ? 0 : r;
   a.n_items = (dq ? r : 0) + (dkdv ? (a.fold_diag ? r / 2 : r) : 0);
   if (a.n_items > bd3::kBwdOrderMax) return;  // the kernel walks the codes in order
@@ -161,6 +200,11 @@ void bwd_order(bd3::BwdArgs& a, bool dq, bool dkdv) {
   }
   std::stable_sort(codes, codes + a.n_items, [&](int x, int y) { return cost[x] > cost[y]; });
   for (int i = 0; i < a.n_items; ++i) a.order[i] = (uint16_t)codes[i];
+  if (dq && dkdv) {
+    int64_t total = 0;
+    for (int i = 0; i < a.n_items; ++i) total += cost[codes[i]];
+    a.subs = bwd_subs(cost[codes[0]], total * a.bh, (int64_t)a.n_items * a.bh);
+  }
 }
 
 // Above this many queries the decode call runs the prefill kernel (128-row
@@ -329,6 +373,7 @@ int bd3_attn_fwd(const void* q, const void* k, const void* v, void* o, float* ls
   a.bh = batch * heads;
   a.n = n;
   a.bs = block_size;
+  a.subs = fwd_subs(a);
   a.scale_log2 = scale * bd3::kLog2e;
   return hip_status(bd3::launch_attn_fwd(a, static_cast<hipStream_t>(stream)), "attn_fwd launch");
 }

@@ -327,3 +327,27 @@ def test_large_logits(cuda, record_error, bs):
     record_error("lse max-abs", max_abs(lse, ref_lse), LSE_TOL)
     for name, got, ref in (("dQ", dq, rdq), ("dK", dk, rdk), ("dV", dv, rdv)):
         record_error(f"{name} rel-F", rel_frobenius(got.cpu(), ref), GRAD_TOL)
+
+
+# Few, long items: two sets of waves share each item's walk. An odd and an even
+# number of tiles per set, a walk of the diagonal tiles alone (n = 512, first
+# rows), a set that meets no key of some rows (block sizes above 64), every
+# mask instance and both backward forms of the noisy diagonal.
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,n,bs", [(1, 2, 512, 16), (1, 1, 640, 5), (1, 1, 640, 128), (2, 1, 768, 4),
+                                      (1, 1, 1024, 1024), (1, 1, 896, 32), (1, 2, 1152, 64)])
+def test_two_wave_sets_match_oracle(cuda, record_error, B, H, n, bs):
+    print(f"two wave sets B={B} H={H} n={n} bs={bs}", flush=True)
+    q, k, v, do = train_inputs(B, H, n, seed=n + bs)
+    qd, kd, vd, dod = to_dev((q, k, v, do), cuda)
+    o, lse = fwd_capi(qd, kd, vd, bs)
+    grads = bwd_capi(qd, kd, vd, o, dod, lse, bs)
+    torch.cuda.synchronize()
+    ref_o, ref_lse = bd3_attention(q, k, v, bs)
+    record_error("O max-abs", max_abs(o, ref_o), OUT_TOL)
+    record_error("lse max-abs", max_abs(lse, ref_lse), LSE_TOL)
+    _, *refs = bd3_attention_grads(q, k, v, do, bs)
+    for name, got, ref in zip(("dQ", "dK", "dV"), grads, refs):
+        record_error(f"{name} rel-F", rel_frobenius(got.cpu(), ref), GRAD_TOL)
+    again = bwd_capi(qd, kd, vd, o, dod, lse, bs)
+    assert all(torch.equal(x, y) for x, y in zip(grads, again))
