@@ -35,11 +35,15 @@
 // more than kRescale (log2 units); otherwise the stale max is kept, which
 // bounds P by 2^kRescale and leaves O / l exact.
 //
-// Few, long items (a.subs = 2): a lone workgroup per CU runs one wave per SIMD,
+// Few, long items (a.subs > 1): a lone workgroup per CU runs one wave per SIMD,
 // and its walk is one chain of load, product, softmax and barrier latencies
 // (~1 us a tile). Two sets of four waves then share the walk, tile by tile in
 // turn, through a ring each, and merge at the end: 1 x 12 heads, n 1024 18.5 ->
-// 15.5 us, n 2048 33.9 -> 28.4 us.
+// 15.5 us, n 2048 33.9 -> 28.4 us. Prefill items are longer still, and two or four
+// sets take the place of key splits with their fp32 partials and merge launch: 1
+// x 12 heads, 3088 queries 39.8 us (4 splits) -> 35.1 (two sets) / 32.4 (four), 4096
+// 57.5 -> 46.7 / 41.6. Four sets (one workgroup a CU) lose for the training forward
+// (1 x 12 heads, n 2048 30.7 us, 3072 55.4 against 29.7 and 45.8 with two).
 //
 // Prefill mode (prefill_attn_kernel, DecodeArgs): the same body over the
 // decode mask when many queries attend to the cache at once (the uncached
@@ -78,8 +82,8 @@ constexpr float kRescale = 8.0f;
 // no mask arithmetic. MASK16: every row's key intervals start and end on
 // multiples of 16 (training: the block size is a multiple of 16; prefill:
 // the block size and kv_len are).
-// SUBS = 2 (training): eight waves, two sets of four that take the walk's tiles
-// in turn, each through a ring of its own; both hold the same rows, and their
+// SUBS = 2, 4: that many sets of four waves, which take the walk's tiles in
+// turn, each through a ring of its own; all hold the same rows, and their
 // (reference, sum, O) are merged at the end.
 template <bool MASK16, bool PREFILL, int SUBS, class Args>
 __device__ __forceinline__ void fwd_body(Args a) {
@@ -87,7 +91,7 @@ __device__ __forceinline__ void fwd_body(Args a) {
   constexpr int kStages = BD3_FWD_STAGES;
   constexpr int kAhead = kStages - 1;  // tiles requested ahead of the one being computed
   __shared__ __attribute__((aligned(1024))) __bf16 smem_all[SUBS][kStages][2][kSwTile];  // [set][stage][K|V]
-  static_assert(SUBS == 1 || (!PREFILL && kStages == 2), "two sets: training, two-stage rings");
+  static_assert(SUBS == 1 || kStages == 2, "several sets: two-stage rings");
 
   const int tid = wi_x();
   const int lane = tid & 63;
@@ -169,21 +173,12 @@ __device__ __forceinline__ void fwd_body(Args a) {
   // made in order: tile_of(0), tile_of(1), ...).
   TileWalk walk(t0, n_first, t2);
   TilePtr kn(kp, 2 * kstep, t0, n_first, t2), vn(vp, 2 * vstep, t0, n_first, t2);
-  // SUBS = 2: walk index i into a stage of the set's ring.
-  auto issue_at = [&](int stage, int i) {
-    const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
-    const int t = wave_uniform(tile_of(i));
-#pragma unroll
-    for (int j = 0; j < 2; ++j) dma16(kp + t * kstep, koff[j], dst + 1024u * j);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) dma16(vp + t * vstep, voff[j], dst + 8192u + 1024u * j);
-  };
-  auto issue = [&](int stage) {
-    const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
-    uint32_t ko[2] = {koff[0], koff[1]}, vo[2] = {voff[0], voff[1]};
+  // Offsets of tile t's rows: those past the last key re-read the last key row
+  // (prefill; masked out).
+  uint32_t ko[2] = {koff[0], koff[1]}, vo[2] = {voff[0], voff[1]};
+  auto clamp_rows = [&](int t) {
     if constexpr (PREFILL) {
-      // Rows past the last key re-read the last key row (masked out).
-      const int lim = a.kv_len - 1 - walk.tile * kSwRows;
+      const int lim = a.kv_len - 1 - t * kSwRows;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int r = imin(lrow[j], lim);
@@ -191,6 +186,20 @@ __device__ __forceinline__ void fwd_body(Args a) {
         vo[j] = (uint32_t)(2 * (r * (int)a.sv.s + lch[j]));
       }
     }
+  };
+  // SUBS > 1: walk index i into a stage of the set's ring.
+  auto issue_at = [&](int stage, int i) {
+    const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
+    const int t = wave_uniform(tile_of(i));
+    clamp_rows(t);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(kp + t * kstep, ko[j], dst + 1024u * j);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) dma16(vp + t * vstep, vo[j], dst + 8192u + 1024u * j);
+  };
+  auto issue = [&](int stage) {
+    const uint32_t dst = lds_w + (uint32_t)stage * 16384u;
+    clamp_rows(walk.tile);
 #pragma unroll
     for (int j = 0; j < 2; ++j) dma16(kn.cur, ko[j], dst + 1024u * j);
 #pragma unroll
@@ -213,12 +222,12 @@ __device__ __forceinline__ void fwd_body(Args a) {
   // the direct loads issued after them, which is harmless.
   bool diag_first = false;
   if constexpr (!PREFILL && kStages == 2) diag_first = q0 < a.n && 32 % a.bs == 0;
-  // SUBS = 2: the set's tiles are walk indices i0, i0 + 2, ...; with the
+  // SUBS > 1: the set's tiles are walk indices i0, i0 + SUBS, ...; with the
   // diagonal step, which set 0 takes, set 1 starts the loop.
   const int n_diag = diag_first ? 2 : 0;
-  const int i0 = n_diag + (diag_first ? 1 - sub : sub);
-  const int n_mine = imax(0, (n_tiles - i0 + 1) >> 1);
-  if constexpr (SUBS == 2) {
+  const int i0 = n_diag + (diag_first ? (sub + SUBS - 1) % SUBS : sub);
+  const int n_mine = imax(0, (n_tiles - i0 + SUBS - 1) / SUBS);
+  if constexpr (SUBS > 1) {
     if (diag_first && sub == 0) {
       issue_at(0, 0);
       issue_at(1, 1);
@@ -448,7 +457,7 @@ __device__ __forceinline__ void fwd_body(Args a) {
     }
   } else {
     if (diag_first) {
-      // As below; set 1 only meets the two barriers.
+      // As above; the other sets only meet the two barriers.
       if (sub == 0) {
         const int st = wave >> 1;
         step(std::integral_constant<int, 1>(), std::true_type(), wave & 1, wave_uniform(tile_of(st) * kSwRows),
@@ -461,10 +470,10 @@ __device__ __forceinline__ void fwd_body(Args a) {
       }
       vm_wait_barrier<0>();
     }
-    const int steps = (n_tiles - n_diag + 1) >> 1;  // of the set with more tiles
+    const int steps = (n_tiles - n_diag + SUBS - 1) / SUBS;  // of the set with the most tiles
     for (int j = 0; j < steps; ++j) {
-      const int i = i0 + 2 * j, cur = j & 1;
-      if (j + 1 < n_mine) issue_at(cur ^ 1, i + 2);
+      const int i = i0 + SUBS * j, cur = j & 1;
+      if (j + 1 < n_mine) issue_at(cur ^ 1, i + SUBS);
       if (j < n_mine && walk_live(wc, i, n_first))
         step(std::integral_constant<int, 2>(), std::false_type(), 0, wave_uniform(tile_of(i) * kSwRows),
              walk_full(wc, i, n_first) ? kFull : kPartial, smem[cur][0], smem[cur][1], [] {});
@@ -473,30 +482,36 @@ __device__ __forceinline__ void fwd_body(Args a) {
   }
 
   float ltot = sum_xor32(lsum);
-  if constexpr (SUBS == 2) {
-    // Set 1 hands its state over through LDS (every wave is past its last read
-    // of the rings); a set that met no key of a row has l = 0.
-    float* ex = reinterpret_cast<float*>(&smem_all[0][0][0][0]) + wave * (34 * 64) + lane;
-    if (sub == 1) {
+  if constexpr (SUBS > 1) {
+    // The other sets hand their state over to set 0 through LDS (every wave is
+    // past its last read of the rings); a set that met no key of a row has l = 0.
+    constexpr int kWave = 34 * 64, kSet = 4 * kWave;
+    static_assert((SUBS - 1) * kSet * 4 <= (int)sizeof(smem_all), "hand-over fits the rings");
+    float* ex = reinterpret_cast<float*>(&smem_all[0][0][0][0]) + wave * kWave + lane;
+    if (sub > 0) {
+      float* my = ex + (sub - 1) * kSet;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        ex[r * 64] = o[0][r];
-        ex[(16 + r) * 64] = o[1][r];
+        my[r * 64] = o[0][r];
+        my[(16 + r) * 64] = o[1][r];
       }
-      ex[32 * 64] = mref;
-      ex[33 * 64] = ltot;
+      my[32 * 64] = mref;
+      my[33 * 64] = ltot;
     }
     __syncthreads();
-    if (sub == 1) return;
-    const float m1 = ex[32 * 64], l1 = ex[33 * 64];
-    const float m = l1 > 0.f ? (ltot > 0.f ? fmaxf(mref, m1) : m1) : mref;
-    const float w0 = ltot > 0.f ? fast_exp2(mref - m) : 0.f, w1 = l1 > 0.f ? fast_exp2(m1 - m) : 0.f;
-    mref = m;
-    ltot = ltot * w0 + l1 * w1;
+    if (sub > 0) return;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      o[0][r] = o[0][r] * w0 + ex[r * 64] * w1;
-      o[1][r] = o[1][r] * w0 + ex[(16 + r) * 64] * w1;
+    for (int t = 0; t < SUBS - 1; ++t, ex += kSet) {
+      const float m1 = ex[32 * 64], l1 = ex[33 * 64];
+      const float m = l1 > 0.f ? (ltot > 0.f ? fmaxf(mref, m1) : m1) : mref;
+      const float w0 = ltot > 0.f ? fast_exp2(mref - m) : 0.f, w1 = l1 > 0.f ? fast_exp2(m1 - m) : 0.f;
+      mref = m;
+      ltot = ltot * w0 + l1 * w1;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        o[0][r] = o[0][r] * w0 + ex[r * 64] * w1;
+        o[1][r] = o[1][r] * w0 + ex[(16 + r) * 64] * w1;
+      }
     }
   }
   if constexpr (PREFILL) {
@@ -544,9 +559,9 @@ __global__ __launch_bounds__(256 * SUBS, OCC) void attn_fwd_dma_kernel(FwdArgs a
   fwd_body<MASK16, false, SUBS>(a);
 }
 
-template <int OCC, bool MASK16>
-__global__ __launch_bounds__(256, OCC) void prefill_attn_kernel(DecodeArgs a) {
-  fwd_body<MASK16, true, 1>(a);
+template <int OCC, bool MASK16, int SUBS>
+__global__ __launch_bounds__(256 * SUBS, OCC) void prefill_attn_kernel(DecodeArgs a) {
+  fwd_body<MASK16, true, SUBS>(a);
 }
 
 // Merges the split partials of the rows whose 128-row tile spans several
@@ -647,11 +662,22 @@ hipError_t launch_prefill(const DecodeArgs& a, hipStream_t stream) {
   // the last key and those a tile does not reach exit at once.
   const int row_tiles = (a.q_len + 127) / 128;
   const int splits = (a.kv_len + a.split_len - 1) / a.split_len;
-  const dim3 grid(a.bh, splits, row_tiles), block(256);
-  if (a.bs % 16 == 0 && a.kv_len % 16 == 0)
-    hipLaunchKernelGGL((prefill_attn_kernel<BD3_FWD_OCC, true>), grid, block, 0, stream, a);
+  const dim3 grid(a.bh, splits, row_tiles), block(256 * a.subs);
+  const bool mask16 = a.bs % 16 == 0 && a.kv_len % 16 == 0;
+  if (a.subs == 4) {
+    if (mask16)
+      hipLaunchKernelGGL((prefill_attn_kernel<4, true, 4>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((prefill_attn_kernel<4, false, 4>), grid, block, 0, stream, a);
+  } else if (a.subs == 2) {
+    if (mask16)
+      hipLaunchKernelGGL((prefill_attn_kernel<4, true, 2>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((prefill_attn_kernel<4, false, 2>), grid, block, 0, stream, a);
+  } else if (mask16)
+    hipLaunchKernelGGL((prefill_attn_kernel<BD3_FWD_OCC, true, 1>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((prefill_attn_kernel<BD3_FWD_OCC, false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((prefill_attn_kernel<BD3_FWD_OCC, false, 1>), grid, block, 0, stream, a);
   hipError_t e = hipGetLastError();
   // The last tile sees the most keys: if they fit one split, no partials.
   if (e != hipSuccess || decode_key_end(128 * (row_tiles - 1), 128, a.q_len, a.kv_len, a.bs) <= a.split_len)

@@ -79,6 +79,7 @@ struct DecodeArgs {
   int bs;
   int n_splits;   // key ranges (workgroups per query tile and batch*head)
   int split_len;  // keys per split (multiple of 32)
+  int subs;       // prefill: sets of 4 waves per workgroup, 1, 2 or 4
   int q_tiles;
   float scale_log2;
 };

@@ -212,7 +212,8 @@ void bwd_order(bd3::BwdArgs& a, bool dq, bool dkdv) {
 // once per 32 rows).
 constexpr int kPrefillMinQ = 65;
 
-// Splits for the prefill kernel: none when the (row tile, batch*head) items
+// The most splits of an automatic prefill call, which sizes its workspace
+// (prefill_plan below takes fewer where that is faster): none when the (row tile, batch*head) items
 // alone fill half of the GPU's workgroup slots (4 per CU on 256 CUs);
 // otherwise as few as keep the longest item (one split of one 128-row tile)
 // under the grid's total work spread over those slots, with kLoneTile = the
@@ -239,6 +240,71 @@ int32_t prefill_auto_splits(int32_t batch, int32_t heads, int32_t q_len, int32_t
   if (s < 1) s = 1;
   if (s > 64) s = 64;
   return (int32_t)s;
+}
+
+// Sets of four waves per workgroup (they share an item's walk, see
+// attn_fwd.hip) and splits of a prefill call.
+struct PrefillPlan {
+  int subs, splits;
+};
+
+// Estimated us of a plan: the longest item's chain against the load per CU.
+// More sets shorten the chain (0.84 / 0.57 / 0.50 us a tile of a lone workgroup
+// with 1 / 2 / 4 sets) at the price of a longer start per item and, with 4 (128
+// KB of LDS), no second workgroup beside it. Splits add the partials' traffic
+// and a merge launch. Constants fitted to 2100 timings, 100 shapes of 65-4096
+// queries, 65-8192 keys and 12-512 heads in all (rms error 9%).
+double prefill_us(int64_t bh, int32_t q_len, int32_t kv_len, int subs, int splits) {
+  struct Cost {
+    double chain0, chain, load0, load, item, merge, partial;
+  };
+  static constexpr Cost kCost[3] = {{2.2, 0.84, 4.4, 0.57, 0.47, 4.4, 0.13},
+                                    {2.7, 0.57, 4.9, 0.55, 1.5, 4.1, 0.125},
+                                    {7.6, 0.50, 5.1, 0.63, 5.8, 4.0, 0.13}};
+  const Cost& c = kCost[subs >> 1];
+  const int split_tiles = ((kv_len + splits - 1) / splits + 63) / 64;
+  int longest = 0;
+  int64_t tiles = 0, items = 0, partials = 0;
+  for (int q0 = 0; q0 < q_len; q0 += 128) {
+    const int t = (kv_len - q_len + std::min(q0 + 128, q_len) + 63) / 64;
+    const int n = splits == 1 ? 1 : (t + split_tiles - 1) / split_tiles;
+    longest = std::max(longest, std::min(t, split_tiles));
+    tiles += t;
+    items += n;
+    partials += n > 1 ? n : 0;
+  }
+  const double cus = 256.0, mb = (double)(partials * bh) * 128 * bd3::kHeadDim * 8 / 1e6;
+  const double chain = c.chain0 + c.chain * longest;
+  const double load = c.load0 + (c.load * (double)tiles + c.item * (double)items) * (double)bh / cus;
+  const double walk = subs == 4 ? std::max(chain, load) : std::sqrt(chain * chain + load * load);
+  return walk + (partials > 0 ? c.merge + c.partial * mb : 0.0);
+}
+
+// The cheapest plan by that estimate; the plain kernel without splits unless
+// another is 5% cheaper. Splitting pays only for few items (at most 128 tried:
+// then a chain cannot be shortened by sets alone), and never with 4 sets. A
+// caller's own split count is taken. us, one set and the earlier split rule ->
+// plan, 12 heads: 1 x 3088 (4 splits) 39.8 -> 32.4 (4 sets), 1 x 4096 57.5 -> 41.6 (4), 2
+// x 2048 35.7 -> 28.0 (2), 4 x 1024 25.6 -> 18.3 (2), 8 x 512 (2 splits) 19.7 -> 12.9 (1),
+// 1 x 128 queries over 4096 keys 14.9 -> 15.4 (1, 16 splits). Over the 100 shapes 11%
+// less time (geometric mean), 0.3% above the best plan of each.
+PrefillPlan prefill_plan(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len, int32_t n_splits,
+                         bool automatic) {
+  constexpr int64_t kSplitItems = 128;
+  const int64_t bh = (int64_t)batch * heads;
+  const int first = automatic ? 1 : n_splits;
+  const int last = !automatic || bh * ((q_len + 127) / 128) <= kSplitItems ? n_splits : 1;
+  PrefillPlan best{1, first};
+  double cost = 0.95 * prefill_us(bh, q_len, kv_len, 1, first);
+  for (int splits = first; splits <= last; ++splits)
+    for (int subs = 1; subs <= (splits == 1 ? 4 : 2); subs *= 2) {
+      const double us = prefill_us(bh, q_len, kv_len, subs, splits);
+      if (us < cost) {
+        cost = us;
+        best = PrefillPlan{subs, splits};
+      }
+    }
+  return best;
 }
 
 int32_t auto_splits(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len) {
@@ -314,6 +380,7 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
   int sl = (kv_len + n_splits - 1) / n_splits;
   sl = (sl + 31) / 32 * 32;
   a.split_len = sl;
+  a.subs = 1;
   a.q_tiles = q_tiles;
   a.scale_log2 = scale * bd3::kLog2e;
   if (q_len >= kPrefillMinQ) {
@@ -323,7 +390,9 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
       const int st = check_dma_stride(strides + 3 * i, i == 1 ? "k" : "v");
       if (st) return st;
     }
-    int pl = (kv_len + n_splits - 1) / n_splits;
+    const PrefillPlan plan = prefill_plan(batch, heads, q_len, kv_len, n_splits, automatic);
+    a.subs = plan.subs;
+    int pl = (kv_len + plan.splits - 1) / plan.splits;
     a.split_len = (pl + 63) / 64 * 64;
     return hip_status(bd3::launch_prefill(a, static_cast<hipStream_t>(stream)), "prefill launch");
   }

@@ -226,7 +226,7 @@ int bd3_decode(const void* q, const void* k, const void* v, void* o,
 
 /*
  * Number of key splits a bd3_decode call is sized for (its workspace; a call
- * of q_len <= 64 uses fewer where that is faster). No reference counterpart.
+ * uses fewer where that is faster). No reference counterpart.
  */
 int32_t bd3_decode_auto_splits(int32_t batch, int32_t heads, int32_t q_len,
                                int32_t kv_len);

@@ -304,3 +304,23 @@ def test_decode_routes_match_oracle(cuda, record_error, B, H, q_len, kv_len, bs,
     for o in (splitkv_capi(dq, dk, dv, bs, n_splits), block_sparse_decode_attention(dq, dk, dv, bs)):
         torch.cuda.synchronize()
         record_error("decode O max-abs", max_abs(o, ref), OUT_TOL)
+
+
+# Prefill calls whose items are shared by two or four sets of waves: tile
+# counts with every remainder, rows that see fewer tiles than there are sets,
+# a ragged last row tile and last key tile, masks per strip and per element;
+# with one split, with splits that keep two sets, and the library's choice.
+WAVE_SETS = [(1, 1, 65, 5000, 16, 1), (1, 1, 129, 5300, 64, 1), (1, 1, 5200, 5200, 5, 1), (1, 2, 4000, 4000, 4, 1),
+             (1, 1, 1000, 1000, 16, 1), (2, 1, 200, 300, 3, 1), (1, 1, 300, 1400, 16, 2), (1, 12, 1600, 3001, 16, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,q_len,kv_len,bs,n_splits", WAVE_SETS)
+def test_prefill_wave_sets_match_oracle(cuda, record_error, B, H, q_len, kv_len, bs, n_splits):
+    print(f"prefill wave sets B={B} H={H} q_len={q_len} kv_len={kv_len} splits={n_splits}", flush=True)
+    q, k, v = decode_inputs(B, H, q_len, kv_len, seed=q_len + kv_len)
+    dq, dk, dv = (t.to(cuda, torch.bfloat16) for t in (q, k, v))
+    ref = decode_attention(q, k, v, bs)
+    for o in (splitkv_capi(dq, dk, dv, bs, n_splits), block_sparse_decode_attention(dq, dk, dv, bs)):
+        torch.cuda.synchronize()
+        record_error("prefill O max-abs (wave sets)", max_abs(o, ref), OUT_TOL)
