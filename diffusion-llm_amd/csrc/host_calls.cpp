@@ -231,12 +231,15 @@ PyObject* attn_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
-// decode(q, k, v, block_size, n_splits) -> O; n_splits 0: bd3_decode's own count
+// decode(q, k, v, block_size, n_splits[, token_major]) -> O; n_splits 0:
+// bd3_decode's own count; token_major: O is a (b, h, s, d) view of (b, s, h, d)
+// memory, so that a caller's transpose + reshape to (b, s, h * d) copies nothing
 PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&] {
-    Args a(args, n, 5);
+    Args a(args, n, n == 6 ? 6 : 5);
     Tensor q = a.tensor(), k = a.tensor(), v = a.tensor();
     const int32_t bs = a.int32(), splits = a.int32();
+    const bool token_major = n == 6 && a.int32() != 0;
     Tensor o;
     {
       NoGil nogil;
@@ -244,8 +247,8 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
       q = ready(q);
       k = ready(k);
       v = ready(v);
-      o = at::empty(q.sizes(), q.options());
       const int32_t B = dim32(q, 0), H = dim32(q, 1), L = dim32(q, 2), D = dim32(q, 3), kv = dim32(k, 2);
+      o = token_major ? at::empty({B, L, H, D}, q.options()).transpose(1, 2) : at::empty(q.sizes(), q.options());
       const size_t bytes = g_lib.decode_workspace_bytes(B, H, L, kv, D, splits);
       const Tensor ws = bytes ? workspace(bytes, q) : Tensor();
       const auto st = strides(q, k, v, o);

@@ -27,13 +27,17 @@ def split_kv_decode_attention(
     """Same result as block_sparse_decode_attention, with the keys split
     across workgroups so a decode step fills the GPU
     (reference: kernels/SplitKVDecodeAttention.py:130-171)."""
-    B, H, q_len, D = q.shape
     kv_len = k.shape[2]
-    if q_len > 64 and n_splits is None:
+    if q.shape[2] > 64 and n_splits is None:
         # prefill: many query tiles already fill the GPU (reference :140-142)
         return block_sparse_decode_attention(q, k, v, block_size)
     _check_decode_inputs(q, k, v)
+    return host().decode(q, k, v, block_size, split_count(kv_len, n_splits))
+
+
+def split_count(kv_len: int, n_splits: int | None) -> int:
+    """n_splits, or the reference's count where it is None."""
     if n_splits is None:
         n_splits = -(-kv_len // SPLIT_N)
     assert 1 <= n_splits <= kv_len, "n_splits must be in [1, kv_len]"
-    return host().decode(q, k, v, block_size, n_splits)
+    return n_splits

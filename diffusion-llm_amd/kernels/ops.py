@@ -9,9 +9,10 @@ carries its backward (register_autograd).
 
     torch.ops.bd3.attn_fwd(q, k, v, block_size) -> (O, L)      differentiable in q, k, v
     torch.ops.bd3.attn_bwd(q, k, v, O, L, dO, block_size) -> (dQ, dK, dV)
-    torch.ops.bd3.decode(q, k, v, block_size, n_splits) -> O   n_splits 0: the library's
-        automatic split (bd3_decode), -1: the reference's split rule (ceil(kv_len / 256),
-        split_kv_decode_attention's default), > 0: that many splits
+    torch.ops.bd3.decode(q, k, v, block_size, n_splits, token_major=False) -> O
+        n_splits 0: the library's automatic split (bd3_decode), -1: the reference's split
+        rule (ceil(kv_len / 256), split_kv_decode_attention's default), > 0: that many
+        splits; token_major: O is a view of (batch, q_len, heads, head_dim) memory
 """
 from __future__ import annotations
 
@@ -76,17 +77,24 @@ attn_fwd.register_autograd(_fwd_backward, setup_context=_fwd_setup_context)
 
 
 @torch.library.custom_op("bd3::decode", mutates_args=())
-def decode(q: Tensor, k: Tensor, v: Tensor, block_size: int, n_splits: int) -> Tensor:
+def decode(q: Tensor, k: Tensor, v: Tensor, block_size: int, n_splits: int, token_major: bool = False) -> Tensor:
     """Block-causal decode of the last q_len positions
     (kernels/BlockSparseDecodeAttention.py:118-148); n_splits > 0 runs the
-    split-KV form (kernels/SplitKVDecodeAttention.py:130-171)."""
-    from kernels.BlockSparseDecodeAttention import block_sparse_decode_attention
-    from kernels.SplitKVDecodeAttention import split_kv_decode_attention
-    if n_splits == 0:
-        return block_sparse_decode_attention(q, k, v, block_size)
-    return split_kv_decode_attention(q, k, v, block_size, n_splits=None if n_splits < 0 else n_splits)
+    split-KV form (kernels/SplitKVDecodeAttention.py:130-171). token_major:
+    O in (batch, q_len, heads, head_dim) memory."""
+    from kernels.BlockSparseDecodeAttention import _check_decode_inputs
+    from kernels.SplitKVDecodeAttention import split_count
+    _check_decode_inputs(q, k, v)
+    if n_splits < 0 and q.shape[2] > 64:
+        n_splits = 0  # prefill: many query tiles already fill the GPU
+    if n_splits != 0:
+        n_splits = split_count(k.shape[2], n_splits if n_splits > 0 else None)
+    return host().decode(q, k, v, block_size, n_splits, int(token_major))
 
 
 @decode.register_fake
-def _decode_fake(q, k, v, block_size, n_splits):
+def _decode_fake(q, k, v, block_size, n_splits, token_major=False):
+    if token_major:
+        B, H, S, Dh = q.shape
+        return q.new_empty((B, S, H, Dh)).transpose(1, 2)
     return q.new_empty(q.shape)

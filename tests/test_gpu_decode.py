@@ -324,3 +324,20 @@ def test_prefill_wave_sets_match_oracle(cuda, record_error, B, H, q_len, kv_len,
     for o in (splitkv_capi(dq, dk, dv, bs, n_splits), block_sparse_decode_attention(dq, dk, dv, bs)):
         torch.cuda.synchronize()
         record_error("prefill O max-abs (wave sets)", max_abs(o, ref), OUT_TOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_len,kv_len,n_splits", [(5, 700, 0), (16, 3000, 0), (32, 1056, 0), (33, 2500, 3), (130, 900, 0),
+                                                   (300, 1400, 4), (16, 700, -1)])
+def test_token_major_result(cuda, q_len, kv_len, n_splits):
+    """The same values, laid out so that the reshape to (b, s, h * d) is a view;
+    every kernel that stores O (one range, merged ranges, prefill and its merge)."""
+    import kernels.ops  # noqa: F401
+    print(f"token major q_len={q_len} kv_len={kv_len} splits={n_splits}", flush=True)
+    B, H = 2, 3
+    q, k, v = (t.to(cuda, torch.bfloat16) for t in decode_inputs(B, H, q_len, kv_len, seed=q_len))
+    plain = torch.ops.bd3.decode(q, k, v, 16, n_splits)
+    o = torch.ops.bd3.decode(q, k, v, 16, n_splits, token_major=True)
+    torch.cuda.synchronize()
+    assert plain.is_contiguous() and o.transpose(1, 2).is_contiguous()
+    assert torch.equal(o, plain)

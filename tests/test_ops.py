@@ -26,3 +26,5 @@ def test_fake_shapes():
         kd = torch.empty(2, 3, 300, 64, dtype=torch.bfloat16)
         od = torch.ops.bd3.decode(qd, kd, kd, 16, 0)
         assert od.shape == qd.shape and od.dtype == torch.bfloat16
+        ot = torch.ops.bd3.decode(qd, kd, kd, 16, 0, token_major=True)
+        assert ot.shape == qd.shape and ot.transpose(1, 2).is_contiguous()
