@@ -286,7 +286,7 @@ double prefill_us(int64_t bh, int32_t q_len, int32_t kv_len, int subs, int split
 // caller's own split count is taken. us, one set and the earlier split rule ->
 // plan, 12 heads: 1 x 3088 (4 splits) 39.8 -> 32.4 (4 sets), 1 x 4096 57.5 -> 41.6 (4), 2
 // x 2048 35.7 -> 28.0 (2), 4 x 1024 25.6 -> 18.3 (2), 8 x 512 (2 splits) 19.7 -> 12.9 (1),
-// 1 x 128 queries over 4096 keys 14.9 -> 15.4 (1, 16 splits). Over the 100 shapes 11%
+// 1 x 128 queries over 4096 keys 15 as before (1, 16 splits). Over the 100 shapes 11%
 // less time (geometric mean), 0.3% above the best plan of each.
 PrefillPlan prefill_plan(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len, int32_t n_splits,
                          bool automatic) {
