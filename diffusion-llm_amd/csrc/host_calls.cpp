@@ -170,6 +170,14 @@ std::array<int64_t, 3 * sizeof...(T)> strides(const T&... ts) {
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
+// The kernels read the operands' addresses as they are: refuses any that is not
+// on the first one's GPU (an undefined one is an absent optional argument).
+template <class... T>
+void on_one_gpu(const Tensor& first, const T&... others) {
+  require(first.is_cuda(), "inputs must be on CUDA");
+  require((... && (!others.defined() || others.device() == first.device())), "inputs must be on one device");
+}
+
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 Tensor workspace(size_t bytes, const Tensor& like) {
@@ -185,6 +193,7 @@ PyObject* attn_fwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Tensor q = a.tensor(), k = a.tensor(), v = a.tensor();
     const int32_t bs = a.int32();
     Tensor o, lse;
+    on_one_gpu(q, k, v);
     {
       NoGil nogil;
       const c10::DeviceGuard device(q.device());
@@ -208,6 +217,7 @@ PyObject* attn_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Tensor q = a.tensor(), k = a.tensor(), v = a.tensor(), o = a.tensor(), lse = a.tensor(), dout = a.tensor();
     const int32_t bs = a.int32();
     Tensor dq, dk, dv;
+    on_one_gpu(q, k, v, o, lse, dout);
     {
       NoGil nogil;
       const c10::DeviceGuard device(q.device());
@@ -241,6 +251,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int32_t bs = a.int32(), splits = a.int32();
     const bool token_major = n == 6 && a.int32() != 0;
     Tensor o;
+    on_one_gpu(q, k, v);
     {
       NoGil nogil;
       const c10::DeviceGuard device(q.device());
@@ -277,6 +288,7 @@ PyObject* qkv_rope(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Tensor k = a.maybe_tensor(), v = a.maybe_tensor();
     const int64_t len = a.integer();
     Tensor q, k_all, v_all;
+    on_one_gpu(qkv, sin, cos, k, v);
     {
       NoGil nogil;
       const c10::DeviceGuard device(qkv.device());
@@ -317,6 +329,7 @@ PyObject* subs_sample(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Tensor u = a.maybe_tensor();
     const uint64_t seed = a.unsigned64(), offset = a.unsigned64();
     Tensor out;
+    on_one_gpu(logits, u);
     {
       NoGil nogil;
       const c10::DeviceGuard device(logits.device());
@@ -364,6 +377,7 @@ PyObject* ln_modulate(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const double eps = a.real();
     const int64_t want = a.integer();
     Tensor out;
+    on_one_gpu(x, w, shift, scale);
     {
       NoGil nogil;
       const c10::DeviceGuard device(x.device());
@@ -389,6 +403,7 @@ PyObject* gate_residual(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&] {
     Args a(args, n, 4);
     Tensor x = a.tensor(), gate = a.tensor(), y = a.tensor(), out = a.maybe_tensor();
+    on_one_gpu(x, gate, y, out);
     {
       NoGil nogil;
       const c10::DeviceGuard device(x.device());
@@ -417,6 +432,7 @@ PyObject* gate_residual_ln_modulate(PyObject*, PyObject* const* args, Py_ssize_t
     const double eps = a.real();
     const int64_t want = a.integer();
     Tensor x_out = a.maybe_tensor(), out;
+    on_one_gpu(x, gate, y, w, shift, scale, x_out);
     {
       NoGil nogil;
       const c10::DeviceGuard device(x.device());

@@ -50,6 +50,9 @@ def _attn_fwd_fake(q, k, v, block_size):
 def attn_bwd(q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor, dout: Tensor,
              block_size: int) -> tuple[Tensor, Tensor, Tensor]:
     """dQ, dK, dV (kernels/BlockSparseFlashAttention.py:508-562)."""
+    _check_train(q, k, v)
+    assert o.shape == dout.shape == q.shape and lse.shape == q.shape[:3], "O, dO and L must match q"
+    assert o.dtype == q.dtype and lse.dtype == torch.float32, "O must be bf16 and L fp32"
     assert (q.shape[2] // 2) % block_size == 0, "n must be a multiple of block_size"
     return host().attn_bwd(q, k, v, o, lse, dout, block_size)
 

@@ -33,6 +33,30 @@ def test_argument_errors_without_a_gpu():
         host.bind({})
 
 
+def test_operands_off_the_gpu_are_refused_without_one():
+    """CPU addresses never reach a launch: the calls raise as they did when
+    the stream was looked up in Python, on a machine with or without a GPU."""
+    import kernels.ops  # noqa: F401
+    host = _native.host()
+    q, lse = torch.zeros(1, 1, 256, 64, dtype=BF), torch.zeros(1, 1, 256)
+    x, m, w = torch.zeros(1, 2, 64, dtype=BF), torch.zeros(1, 64, dtype=BF), torch.zeros(64, dtype=BF)
+    qkv, table = torch.zeros(1, 4, 192, dtype=BF), torch.zeros(8, 32)
+    block = torch.zeros(1, 2, dtype=torch.int64)
+    for call in (
+        lambda: torch.ops.bd3.attn_bwd(q, q, q, q, lse, q, 16),
+        lambda: host.attn_fwd(q, q, q, 16),
+        lambda: host.attn_bwd(q, q, q, q, lse, q, 16),
+        lambda: host.decode(q, q, q, 16, 0),
+        lambda: host.qkv_rope(qkv, 1, table, table, None, 0, None, None, 0),
+        lambda: host.subs_sample(x, block, 63, 0.5, None, 0, 0),
+        lambda: host.ln_modulate(x, w, m, m, 1e-5, -1),
+        lambda: host.gate_residual(x, m, x, None),
+        lambda: host.gate_residual_ln_modulate(x, m, x, w, m, m, 1e-5, -1, None),
+    ):
+        with pytest.raises(AssertionError, match="CUDA"):
+            call()
+
+
 def rnd(dev, *shape, seed=0, dtype=BF):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dev, dtype)
 
@@ -103,6 +127,40 @@ def test_refusals_keep_their_types(cuda):
         ln_modulate(x.half(), m[0], m, m)
     with pytest.raises(KeyError):
         ln_modulate(x, m[0], m, m, out_dtype=torch.float16)
+
+
+@pytest.mark.gpu
+def test_one_operand_off_the_gpu_is_refused(cuda):
+    """Every operand is looked at, not the first alone; the backward op also
+    refuses the shapes and dtypes its forward would not have saved."""
+    import kernels.ops  # noqa: F401
+    q, lse = rnd(cuda, 1, 1, 256, 64), torch.zeros(1, 1, 256, device=cuda)
+    x, m, w = rnd(cuda, 2, 5, 64), rnd(cuda, 2, 64), rnd(cuda, 64)
+    sin, cos = rope_tables(64, 32, device=cuda)
+    block = torch.full((2, 5), 63, device=cuda)
+
+    def train(q, k, v, o, lse, do):
+        return torch.ops.bd3.attn_bwd(q, k, v, o, lse, do, 16)
+
+    calls = [
+        (train, (q, q, q, q, lse, q)),
+        (lambda *a: BlockSparseFlashAttention.apply(*a, 16), (q, q, q)),
+        (lambda *a: block_sparse_decode_attention(*a, 16), (q, q, q)),
+        (lambda *a: split_kv_decode_attention(*a, 16, n_splits=2), (q, q, q)),
+        (lambda qkv, s, c: attention_inputs(qkv, 1, s, c), (rnd(cuda, 1, 4, 192), sin, cos)),
+        (lambda *a: ln_modulate(*a), (x, w, m, m)),
+        (lambda *a: gate_residual(*a), (x, m, x, x.clone())),
+        (lambda *a: gate_residual_ln_modulate(*a), (x, m, x, w, m, m)),
+        (lambda lg, u: subs_sample_step(lg, block, 63, 0.5, u=u), (x, torch.rand(2, 5, 64, device=cuda).double())),
+    ]
+    for call, args in calls:
+        for i in range(len(args)):
+            with pytest.raises(AssertionError):
+                call(*(a.cpu() if i == j else a for j, a in enumerate(args)))
+    for bad in ((q, q, q, q.float(), lse, q), (q, q, q, q, lse.double(), q), (q, q, q, q, lse[..., :128], q),
+                (q, q[:, :, :128], q, q, lse, q), (q.half(), q, q, q, lse, q), (q, q, q, q, lse, q[:, :, :128])):
+        with pytest.raises(AssertionError):
+            train(*bad)
 
 
 @pytest.mark.gpu
