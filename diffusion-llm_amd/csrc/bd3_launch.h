@@ -147,6 +147,14 @@ struct GlueArgs {
   int wave_rows, wg_threads;  // set at the launch: rows per wave, threads per workgroup
 };
 
+// Launch shape of the kernels that walk rows (ln_modulate, the fused one);
+// workgroups 0: more threads than a launch holds.
+struct GlueGrid {
+  int wave_rows, threads;
+  unsigned workgroups;
+};
+GlueGrid glue_grid(int rows, int d);
+
 hipError_t launch_attn_fwd(const FwdArgs& a, hipStream_t stream);
 // The backward's Delta pass (Delta and -L / scale), then one launch of the
 // items in a.order (dQ and / or dK/dV).

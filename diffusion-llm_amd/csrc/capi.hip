@@ -927,6 +927,17 @@ int bd3_gate_residual_ln_modulate(const void* x, int32_t x_fp32, const void* gat
                     "gate_residual_ln_modulate launch");
 }
 
+int bd3_glue_grid(int32_t rows, int32_t d_model, int64_t* out) {
+  if (rows < 1 || d_model < 8 || d_model % 8 != 0 || d_model > 4096 || out == nullptr)
+    return fail(BD3_EINVAL, "rows >= 1, d_model a multiple of 8 up to 4096 and a non-NULL out are needed");
+  const bd3::GlueGrid g = bd3::glue_grid(rows, d_model);
+  if (g.workgroups == 0) return fail(BD3_EINVAL, "%d rows of %d do not fit a launch", rows, d_model);
+  out[0] = g.wave_rows;
+  out[1] = g.threads;
+  out[2] = g.workgroups;
+  return BD3_OK;
+}
+
 int bd3_mask_dump(uint8_t* out, int32_t mode, int32_t rows, int32_t kv_len, int32_t block_size,
                   void* stream) {
   if (out == nullptr) return fail(BD3_EINVAL, "out is NULL");

@@ -137,9 +137,10 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
   constexpr bool kModBf16 = !kRowF32 && !MF;             // modulate in bf16 iff the row and the vectors are
   const int lane = wi_x() & 63;
   const int wave = wave_uniform((int)(wg_x() * (a.wg_threads >> 6) + (wi_x() >> 6)));
-  const int r0 = wave * a.wave_rows;
-  const int r1 = imin(a.rows, r0 + a.wave_rows);
-  if (r0 >= r1) return;
+  // unsigned: the last workgroup's waves may start past 2^31 (at most 2^25 + 3 waves of 64 rows)
+  const uint32_t first = (uint32_t)wave * (uint32_t)a.wave_rows;
+  if (first >= (uint32_t)a.rows) return;
+  const int r0 = (int)first, r1 = r0 + imin(a.wave_rows, a.rows - r0);
   const int nch = a.d >> 2;
   const float d_inv = (float)a.d;
   int col[CH];  // first element of the lane's chunk k (lanes past the row repeat its last chunk)
@@ -386,6 +387,29 @@ __global__ __launch_bounds__(256) void gate_residual_kernel(GlueArgs a) {
 }  // namespace
 
 namespace {
+// 4-element chunks of a row per lane.
+int glue_chunks(int d) { return (d / 4 + 63) / 64; }
+}  // namespace
+
+// Rows per wave: enough waves to keep 8 per SIMD (8192 over 1024 SIMDs), then
+// up to 8 rows each, so that the vectors are loaded once for them and the
+// next row is on its way. 8 x 2048 rows x 768 (fp32 residual): fused 31.1 us at
+// 2 rows a wave, 32.5 at 4, 34.4 at 8, 31.9 at 1; alone 12.9 / 12.8 / 13.6 /
+// 13.8. Few rows take one-wave workgroups, which spread over all CUs. A launch
+// holds fewer than 2^32 threads: very many rows take more than 8 a wave, and
+// where a wave holds one row (d_model > 1024) more than 2^26 - 4 are refused.
+GlueGrid glue_grid(int rows, int d) {
+  GlueGrid g;
+  const bool several = glue_chunks(d) <= 4;
+  g.wave_rows = several ? imax(imin(imax(rows / 8192, 1), 8), (int)(((int64_t)rows + (1 << 25) - 1) >> 25)) : 1;
+  const int64_t waves = ((int64_t)rows + g.wave_rows - 1) / g.wave_rows;
+  g.threads = waves <= 1024 ? 64 : 256;
+  const int64_t per = g.threads / 64, workgroups = (waves + per - 1) / per;
+  g.workgroups = workgroups * g.threads <= (int64_t)UINT32_MAX ? (unsigned)workgroups : 0;
+  return g;
+}
+
+namespace {
 
 template <int CH, bool FUSED>
 void launch_rows_ch(const GlueArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
@@ -410,17 +434,13 @@ void launch_rows_ch(const GlueArgs& a, dim3 grid, dim3 block, hipStream_t stream
 template <bool FUSED>
 hipError_t launch_rows(GlueArgs a, hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
-  const int ch = (a.d / 4 + 63) / 64;  // 4-element chunks per lane
+  const int ch = glue_chunks(a.d);
   if (ch > 16) return hipErrorInvalidValue;  // d_model > 4096: rejected by the C ABI
-  // Rows per wave: enough waves to keep 8 per SIMD (8192 over 1024 SIMDs), then
-  // up to 8 rows each, so that the vectors are loaded once for them and the
-  // next row is on its way. 8 x 2048 rows x 768 (fp32 residual): fused 31.1 us at
-  // 2 rows a wave, 32.5 at 4, 34.4 at 8, 31.9 at 1; alone 12.9 / 12.8 / 13.6 /
-  // 13.8. Few rows take one-wave workgroups, which spread over all CUs.
-  a.wave_rows = ch <= 4 ? imin(imax(a.rows / 8192, 1), 8) : 1;
-  const int waves = (a.rows + a.wave_rows - 1) / a.wave_rows;
-  a.wg_threads = waves <= 1024 ? 64 : 256;
-  const dim3 block(a.wg_threads), grid((unsigned)((waves * 64 + a.wg_threads - 1) / a.wg_threads));
+  const GlueGrid g = glue_grid(a.rows, a.d);
+  if (g.workgroups == 0) return hipErrorInvalidValue;
+  a.wave_rows = g.wave_rows;
+  a.wg_threads = g.threads;
+  const dim3 block(g.threads), grid(g.workgroups);
   if (ch <= 1)
     launch_rows_ch<1, FUSED>(a, grid, block, stream);
   else if (ch <= 2)

@@ -408,6 +408,14 @@ int bd3_gate_residual_ln_modulate(const void* x, int32_t x_fp32, const void* gat
                                   void* stream);
 
 /*
+ * Launch shape of bd3_ln_modulate / bd3_gate_residual_ln_modulate for rows =
+ * batch * seq (host only, for tests): out[0] rows per 64-thread wave, out[1]
+ * threads per workgroup, out[2] workgroups. BD3_EINVAL where the rows do not
+ * fit a launch. No reference counterpart.
+ */
+int bd3_glue_grid(int32_t rows, int32_t d_model, int64_t* out);
+
+/*
  * Writes the mask the device predicate applies, one byte per (row, key)
  * (1 = may attend), row-major:
  *   mode 0 (training): (2n, 2n) with n = rows, kv_len ignored;
