@@ -145,12 +145,13 @@ struct GlueArgs {
   int64_t sx_b, sx_s, sm_b, sy_b, sy_s, so_b, so_s, sxo_b, sxo_s;  // element strides
   float eps;
   int wave_rows, wg_threads;  // set at the launch: rows per wave, threads per workgroup
+  int row0;                   // first row of the launch (rows: the one past its last)
 };
 
-// Launch shape of the kernels that walk rows (ln_modulate, the fused one);
-// workgroups 0: more threads than a launch holds.
+// Launch shape of the kernels that walk rows (ln_modulate, the fused one), for
+// each launch of `rows` rows (the last may have fewer).
 struct GlueGrid {
-  int wave_rows, threads;
+  int wave_rows, threads, rows;
   unsigned workgroups;
 };
 GlueGrid glue_grid(int rows, int d);

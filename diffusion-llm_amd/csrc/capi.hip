@@ -931,10 +931,10 @@ int bd3_glue_grid(int32_t rows, int32_t d_model, int64_t* out) {
   if (rows < 1 || d_model < 8 || d_model % 8 != 0 || d_model > 4096 || out == nullptr)
     return fail(BD3_EINVAL, "rows >= 1, d_model a multiple of 8 up to 4096 and a non-NULL out are needed");
   const bd3::GlueGrid g = bd3::glue_grid(rows, d_model);
-  if (g.workgroups == 0) return fail(BD3_EINVAL, "%d rows of %d do not fit a launch", rows, d_model);
   out[0] = g.wave_rows;
   out[1] = g.threads;
   out[2] = g.workgroups;
+  out[3] = g.rows;
   return BD3_OK;
 }
 

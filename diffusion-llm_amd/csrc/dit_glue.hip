@@ -20,12 +20,14 @@
 //   lanes of a 768-wide row were idle and every row reloaded its vectors (6 KB
 //   against the row's own 4.5). 8 x 2048 x 768, fp32 x, bf16 result: 17.2 ->
 //   12.9 us (5.9 TB/s); FUSED 37.6 -> 31.1 us (4.9 TB/s); bf16 x: 16.7 -> 11.8
-//   and 29.3 -> 23.4 us; 4096 x 2048 fp32: 15.9 -> 12.4 and 26.4 -> 23.5 us; 1024
-//   x 4096: 12.7 -> 9.4 and 17.3 -> 13.6 us.
+//   and 29.3 -> 23.4 us; 4096 x 2048 fp32: 15.9 -> 12.4 and 26.4 -> 23.5 us. Two
+//   waves to a row above 2048 features: see ln_modulate_kernel.
 // gate_residual_kernel: x + gate * y (the residual updates of
 //   DiTBlock.forward, :560-566): gate * y in the promoted dtype of gate and y,
 //   then the add in the promoted dtype of x and that product; bit-exact with
 //   the eager ops. out may alias x.
+#include <algorithm>
+
 #include "bd3_device.h"
 #include "bd3_launch.h"
 #include "bd3_mask.h"
@@ -124,28 +126,39 @@ __device__ __forceinline__ void store4(void* p, bool fp32, const float (&v)[4]) 
 //
 // A wave owns `a.wave_rows` consecutive rows; lane l holds the 4-element chunks
 // l, l + 64, ... of a row, so every load and store of a wave is one contiguous
-// piece. CH: chunks per lane (d_model <= 256 * CH). Rows of up to 4 chunks per
+// piece. CH: chunks per lane. Rows of up to 4 chunks per
 // lane keep the gain, 1 + scale and shift (and the gate) in registers from row
 // to row and request the next row before they work on the current one; longer
 // rows load them per row. XF / MF / YF: x, the vectors, y in fp32.
-template <int CH, bool XF, bool MF, bool YF, bool FUSED>
-__global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
+//
+// PAIR: rows of more than 2048, two waves (a 128-thread workgroup) to a row,
+// each with every other run of 64 chunks, and the sums exchanged through LDS:
+// 126-228 VGPRs, two to four waves per SIMD. One wave a row would hold up to 16
+// chunks per lane (246-256 VGPRs and up to 184 AGPRs, one or two waves per SIMD).
+// us with one -> two waves, bf16 result, x / vectors: 16384 x 2304 bf16 / fp32 76.8
+// -> 37.5, bf16 / bf16 FUSED 136.9 -> 76.7; 16384 x 4096 fp32 / bf16 87.0 -> 82.5,
+// FUSED 182 -> 152, bf16 / bf16 FUSED 176 -> 110; 1024 x 4096 fp32 / bf16 8.4 (8.4),
+// FUSED 14.3 -> 13.4.
+template <int CH, bool XF, bool MF, bool YF, bool FUSED, bool PAIR>
+__global__ __launch_bounds__(PAIR ? 128 : 256) void ln_modulate_kernel(GlueArgs a) {
 #pragma clang fp contract(off)  // separate products and sums, as the eager ops
+  static_assert(!PAIR || CH > 4, "shorter rows keep their vectors");
+  constexpr int kStep = PAIR ? 128 : 64;  // chunks between a lane's chunks
   constexpr bool KEEP = CH <= 4;
   constexpr bool kGyBf16 = !MF && !YF;
   constexpr bool kRowF32 = FUSED ? XF || MF || YF : XF;  // dtype of the row that is normalised
   constexpr bool kModBf16 = !kRowF32 && !MF;             // modulate in bf16 iff the row and the vectors are
-  const int lane = wi_x() & 63;
-  const int wave = wave_uniform((int)(wg_x() * (a.wg_threads >> 6) + (wi_x() >> 6)));
+  const int lane = PAIR ? wi_x() : wi_x() & 63;  // in the row
+  const int wave = PAIR ? wg_x() : wave_uniform((int)(wg_x() * (a.wg_threads >> 6) + (wi_x() >> 6)));
   // unsigned: the last workgroup's waves may start past 2^31 (at most 2^25 + 3 waves of 64 rows)
-  const uint32_t first = (uint32_t)wave * (uint32_t)a.wave_rows;
+  const uint32_t first = (uint32_t)a.row0 + (uint32_t)wave * (uint32_t)a.wave_rows;
   if (first >= (uint32_t)a.rows) return;
   const int r0 = (int)first, r1 = r0 + imin(a.wave_rows, a.rows - r0);
   const int nch = a.d >> 2;
   const float d_inv = (float)a.d;
   int col[CH];  // first element of the lane's chunk k (lanes past the row repeat its last chunk)
 #pragma unroll
-  for (int k = 0; k < CH; ++k) col[k] = 4 * imin(lane + 64 * k, nch - 1);
+  for (int k = 0; k < CH; ++k) col[k] = 4 * imin(lane + kStep * k, nch - 1);
 
   auto x_row = [&](int b, int s) { return elem(a.x, XF, (int64_t)b * a.sx_b + (int64_t)s * a.sx_s); };
   auto y_row = [&](int b, int s) { return elem(a.y, YF, (int64_t)b * a.sy_b + (int64_t)s * a.sy_s); };
@@ -219,6 +232,19 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
       vs[k].load(elem(a.shift, MF, (int64_t)b * a.sm_b + col[k]));
     }
   }
+  // Sum over the row's lanes. PAIR: of the two waves' sums, an LDS slot for each
+  // and for each of the row's two sums.
+  __shared__ float part[2][2];
+  auto row_sum = [&](float v, int use) {
+    v = wave_sum(v);
+    if constexpr (PAIR) {
+      const int half = (int)wi_x() >> 6;
+      if ((wi_x() & 63) == 0) part[use][half] = v;
+      __syncthreads();
+      v += part[use][half ^ 1];
+    }
+    return v;
+  };
 
   for (int row = r0;;) {
     // the row's values (zero past its end); with FUSED the updated residual, stored
@@ -235,7 +261,7 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
         } else {
           vg[k].get(gv);
         }
-        const bool in = lane + 64 * k < nch;
+        const bool in = lane + kStep * k < nch;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float gy = gv[e] * yv[e];
@@ -249,7 +275,7 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         xr[k].get(v[k]);
-        const bool in = lane + 64 * k < nch;
+        const bool in = lane + kStep * k < nch;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[k][e] = in ? v[k][e] : 0.f;
       }
@@ -268,11 +294,11 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
     for (int k = 0; k < CH; ++k)
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum += v[k][e];
-    const float mean = wave_sum(sum) / d_inv;
+    const float mean = row_sum(sum, 0) / d_inv;
     float sq = 0.f;
 #pragma unroll
     for (int k = 0; k < CH; ++k) {
-      const bool in = lane + 64 * k < nch;
+      const bool in = lane + kStep * k < nch;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         v[k][e] -= mean;
@@ -280,7 +306,7 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
         sq += in ? dd : 0.f;
       }
     }
-    const float inv = rsqrtf(wave_sum(sq) / d_inv + a.eps);
+    const float inv = rsqrtf(row_sum(sq, 1) / d_inv + a.eps);
     char* outr = const_cast<char*>(elem(a.out, a.out_fp32, (int64_t)b * a.so_b + (int64_t)s * a.so_s));
 #pragma unroll
     for (int k = 0; k < CH; ++k) {
@@ -303,7 +329,7 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(GlueArgs a) {
         const float te = KEEP ? t[KEEP ? k : 0][e] : tk[e], se = KEEP ? sh[KEEP ? k : 0][e] : shk[e];
         o[e] = kModBf16 ? rbf(rbf(y * te) + se) : y * te + se;
       }
-      if (lane + 64 * k < nch) store4(outr + (int64_t)col[k] * (a.out_fp32 ? 4 : 2), a.out_fp32, o);
+      if (lane + kStep * k < nch) store4(outr + (int64_t)col[k] * (a.out_fp32 ? 4 : 2), a.out_fp32, o);
     }
     if (!KEEP || nrow >= r1) break;
     if constexpr (KEEP)
@@ -387,8 +413,9 @@ __global__ __launch_bounds__(256) void gate_residual_kernel(GlueArgs a) {
 }  // namespace
 
 namespace {
+bool glue_pair(int d) { return d > 2048; }  // two waves to a row
 // 4-element chunks of a row per lane.
-int glue_chunks(int d) { return (d / 4 + 63) / 64; }
+int glue_chunks(int d) { return (d / 4 + (glue_pair(d) ? 127 : 63)) / (glue_pair(d) ? 128 : 64); }
 }  // namespace
 
 // Rows per wave: enough waves to keep 8 per SIMD (8192 over 1024 SIMDs), then
@@ -396,24 +423,25 @@ int glue_chunks(int d) { return (d / 4 + 63) / 64; }
 // next row is on its way. 8 x 2048 rows x 768 (fp32 residual): fused 31.1 us at
 // 2 rows a wave, 32.5 at 4, 34.4 at 8, 31.9 at 1; alone 12.9 / 12.8 / 13.6 /
 // 13.8. Few rows take one-wave workgroups, which spread over all CUs. A launch
-// holds fewer than 2^32 threads: very many rows take more than 8 a wave, and
-// where a wave holds one row (d_model > 1024) more than 2^26 - 4 are refused.
+// holds fewer than 2^32 threads: very many short rows take more than 8 a wave,
+// longer ones go out in launches of 2^24.
 GlueGrid glue_grid(int rows, int d) {
   GlueGrid g;
   const bool several = glue_chunks(d) <= 4;
+  g.rows = several ? rows : imin(rows, 1 << 24);
   g.wave_rows = several ? imax(imin(imax(rows / 8192, 1), 8), (int)(((int64_t)rows + (1 << 25) - 1) >> 25)) : 1;
-  const int64_t waves = ((int64_t)rows + g.wave_rows - 1) / g.wave_rows;
-  g.threads = waves <= 1024 ? 64 : 256;
-  const int64_t per = g.threads / 64, workgroups = (waves + per - 1) / per;
-  g.workgroups = workgroups * g.threads <= (int64_t)UINT32_MAX ? (unsigned)workgroups : 0;
+  const int64_t waves = ((int64_t)g.rows + g.wave_rows - 1) / g.wave_rows;
+  g.threads = glue_pair(d) ? 128 : waves <= 1024 ? 64 : 256;
+  const int64_t per = glue_pair(d) ? 1 : g.threads / 64;  // waves (pairs of them) per workgroup
+  g.workgroups = (unsigned)((waves + per - 1) / per);
   return g;
 }
 
 namespace {
 
-template <int CH, bool FUSED>
+template <int CH, bool FUSED, bool PAIR = false>
 void launch_rows_ch(const GlueArgs& a, dim3 grid, dim3 block, hipStream_t stream) {
-#define BD3_ROWS(XF, MF, YF) hipLaunchKernelGGL((ln_modulate_kernel<CH, XF, MF, YF, FUSED>), grid, block, 0, stream, a)
+#define BD3_ROWS(XF, MF, YF) hipLaunchKernelGGL((ln_modulate_kernel<CH, XF, MF, YF, FUSED, PAIR>), grid, block, 0, stream, a)
   const int t = (a.x_fp32 ? 4 : 0) | (a.m_fp32 ? 2 : 0) | (FUSED && a.y_fp32 ? 1 : 0);
   switch (t) {
     case 0: BD3_ROWS(false, false, false); break;
@@ -435,26 +463,31 @@ template <bool FUSED>
 hipError_t launch_rows(GlueArgs a, hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
   const int ch = glue_chunks(a.d);
-  if (ch > 16) return hipErrorInvalidValue;  // d_model > 4096: rejected by the C ABI
+  if (ch > 8) return hipErrorInvalidValue;  // d_model > 4096: rejected by the C ABI
   const GlueGrid g = glue_grid(a.rows, a.d);
-  if (g.workgroups == 0) return hipErrorInvalidValue;
   a.wave_rows = g.wave_rows;
   a.wg_threads = g.threads;
   const dim3 block(g.threads), grid(g.workgroups);
-  if (ch <= 1)
-    launch_rows_ch<1, FUSED>(a, grid, block, stream);
-  else if (ch <= 2)
-    launch_rows_ch<2, FUSED>(a, grid, block, stream);
-  else if (ch <= 3)
-    launch_rows_ch<3, FUSED>(a, grid, block, stream);
-  else if (ch <= 4)
-    launch_rows_ch<4, FUSED>(a, grid, block, stream);
-  else if (ch <= 6)
-    launch_rows_ch<6, FUSED>(a, grid, block, stream);
-  else if (ch <= 8)
-    launch_rows_ch<8, FUSED>(a, grid, block, stream);
-  else
-    launch_rows_ch<16, FUSED>(a, grid, block, stream);
+  const int rows = a.rows;
+  for (int64_t r = 0; r < rows; r += g.rows) {
+    a.row0 = (int)r;
+    a.rows = (int)std::min<int64_t>(rows, r + g.rows);  // the launch's end
+    if (glue_pair(a.d))
+      ch <= 6 ? launch_rows_ch<6, FUSED, true>(a, grid, block, stream)
+              : launch_rows_ch<8, FUSED, true>(a, grid, block, stream);
+    else if (ch <= 1)
+      launch_rows_ch<1, FUSED>(a, grid, block, stream);
+    else if (ch <= 2)
+      launch_rows_ch<2, FUSED>(a, grid, block, stream);
+    else if (ch <= 3)
+      launch_rows_ch<3, FUSED>(a, grid, block, stream);
+    else if (ch <= 4)
+      launch_rows_ch<4, FUSED>(a, grid, block, stream);
+    else if (ch <= 6)
+      launch_rows_ch<6, FUSED>(a, grid, block, stream);
+    else
+      launch_rows_ch<8, FUSED>(a, grid, block, stream);
+  }
   return hipGetLastError();
 }
 

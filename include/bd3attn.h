@@ -409,9 +409,9 @@ int bd3_gate_residual_ln_modulate(const void* x, int32_t x_fp32, const void* gat
 
 /*
  * Launch shape of bd3_ln_modulate / bd3_gate_residual_ln_modulate for rows =
- * batch * seq (host only, for tests): out[0] rows per 64-thread wave, out[1]
- * threads per workgroup, out[2] workgroups. BD3_EINVAL where the rows do not
- * fit a launch. No reference counterpart.
+ * batch * seq (host only, for tests): out[0] rows per wave (d_model > 2048: per
+ * pair of waves), out[1] threads per workgroup, out[2] workgroups, out[3] rows
+ * per launch (more rows go out in several). No reference counterpart.
  */
 int bd3_glue_grid(int32_t rows, int32_t d_model, int64_t* out);
 

@@ -426,28 +426,25 @@ def test_subs_sample_workspace_validation(lib):
     assert call(p, need, mask=50258) == _native.BD3_EINVAL and "mask_index" in _native.last_error()
 
 
-@pytest.mark.parametrize("d", [8, 768, 1024, 1032, 4096])
-@pytest.mark.parametrize("rows", [1, 3, 1024, 1025, 16384, 65537, (1 << 25) - 1, 1 << 25, (1 << 25) + 1, (1 << 26) - 4,
-                                  (1 << 26) - 3, (1 << 28) + 1, (1 << 29) + 8192, (1 << 31) - 1])
+@pytest.mark.parametrize("d", [8, 768, 1024, 1032, 2048, 2056, 4096])
+@pytest.mark.parametrize("rows", [1, 3, 1024, 1025, 16384, 65537, (1 << 24) + 1, (1 << 25) - 1, 1 << 25, (1 << 25) + 1,
+                                  (1 << 26) - 4, (1 << 28) + 1, (1 << 29) + 8192, (1 << 31) - 1])
 def test_glue_grid_covers_the_rows(lib, rows, d):
-    """Every row has a wave, no workgroup is without one, and a launch stays
-    below 2^32 threads, up to the most rows the C ABI takes; what one launch
-    cannot hold (a row per wave) is refused and not cut short."""
-    out = (ctypes.c_int64 * 3)()
-    status = lib.bd3_glue_grid(rows, d, out)
-    if d > 1024 and rows > (1 << 26) - 4:
-        expect_einval(status, "do not fit")
-        return
-    assert status == 0
-    wave_rows, threads, workgroups = out
-    per = wave_rows * (threads // 64)
-    assert (workgroups - 1) * per < rows <= workgroups * per
+    """Every row of a launch has a wave (above 2048 features a pair of them),
+    no workgroup is without one, and a launch stays below 2^32 threads, up to
+    the most rows the C ABI takes."""
+    out = (ctypes.c_int64 * 4)()
+    assert lib.bd3_glue_grid(rows, d, out) == 0
+    wave_rows, threads, workgroups, at_once = out
+    assert at_once == (rows if d <= 1024 else min(rows, 1 << 24))
+    per = wave_rows * (threads // (64 if d <= 2048 else 128))
+    assert (workgroups - 1) * per < at_once <= workgroups * per
     assert workgroups * threads < 1 << 32
-    # the kernel forms a wave's first row as an unsigned 32-bit product
-    assert workgroups * per < 1 << 32 and wave_rows <= (64 if d <= 1024 else 1)
+    # the kernel forms a wave's first row as an unsigned 32-bit sum and product
+    assert rows + workgroups * per < 1 << 32 and wave_rows <= (64 if d <= 1024 else 1)
 
 
 def test_glue_grid_validation(lib):
-    out = (ctypes.c_int64 * 3)()
+    out = (ctypes.c_int64 * 4)()
     for rows, d, o in ((0, 768, out), (1, 4, out), (1, 100, out), (1, 4104, out), (1, 768, None)):
         expect_einval(lib.bd3_glue_grid(rows, d, o), "rows >= 1")

@@ -26,9 +26,8 @@ def rnd(shape, dtype, seed, scale=1.0, shift=0.0):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("xd,md,od", [(F32, BF, F32), (F32, BF, BF), (BF, BF, BF), (BF, F32, F32), (F32, F32, F32)])
-# Rows per wave: 4 up to d = 1024, 2 up to 2048, 1 beyond; sequence lengths
-# that are not multiples of that put two batch indices in one wave; d = 520
-# leaves one lane with a second, last chunk.
+# One row a wave (two waves a row at d = 4096; several rows a wave: below); d =
+# 520 leaves two lanes with a third, last chunk.
 @pytest.mark.parametrize("B,S,D", [(2, 37, 768), (1, 5, 64), (8, 256, 768), (2, 9, 2048), (3, 7, 4096),
                                    (2, 11, 520)])
 def test_ln_modulate(cuda, xd, md, od, B, S, D):
@@ -134,3 +133,31 @@ def test_several_rows_per_wave(cuda, xd, B, S, D):
     diff = (got_h.float() - want).abs()
     assert (diff <= 3 * 2.0 ** -7 * mag + 1e-30).all(), float((diff / (mag + 1e-30)).max())
     assert (diff > 0).float().mean() < 0.01, float((diff > 0).float().mean())
+
+
+@pytest.mark.gpu
+# Two waves to a row. 2056: one lane of the first wave with a fifth chunk and
+# none of the second; 2304: half of the first wave; 3072: six chunks a lane;
+# 3080, 4088: a seventh, an eighth not in every lane.
+@pytest.mark.parametrize("D", [2056, 2304, 3072, 3080, 4088])
+def test_rows_of_two_waves(cuda, D):
+    for xd, md, od in ((F32, BF, F32), (F32, BF, BF), (BF, BF, BF), (BF, F32, F32), (F32, F32, F32)):
+        test_ln_modulate(cuda, xd, md, od, 3, 5, D)
+    for xd, md, yd, od in ((BF, BF, BF, BF), (F32, BF, BF, None), (BF, F32, BF, None), (F32, F32, F32, None),
+                           (BF, BF, F32, None), (BF, F32, F32, None), (F32, BF, F32, None), (F32, F32, BF, None)):
+        test_gate_residual_ln_modulate_matches_two_calls(cuda, xd, md, yd, od, 3, 5, D)
+
+
+@pytest.mark.gpu
+# 2^24 + 4096 rows of 1032 and of 2056 (two launches; one and two waves a row), 2^29
+# + 8192 of 8 (17 rows a wave; waves * 64 does not fit 32 bits).
+@pytest.mark.parametrize("B,S,D", [(4097, 4096, 1032), (4097, 4096, 2056), (131074, 4096, 8)])
+def test_very_many_rows(cuda, B, S, D):
+    """One sequence repeated by a batch stride of 0: every entry of the
+    result is the first one's, which a call of one sequence gives."""
+    print(f"rows {B} x {S} x {D}", flush=True)
+    x, w, m = rnd((1, S, D), BF, 31).to(cuda), rnd((D,), F32, 32).to(cuda), rnd((1, D), BF, 33).to(cuda)
+    want = ln_modulate(x, w, m, m)
+    got = ln_modulate(x.expand(B, S, D), w, m.expand(B, D), m.expand(B, D))
+    for b in range(0, B, 256):
+        assert torch.equal(got[b:b + 256], want.expand(min(256, B - b), S, D)), b
