@@ -248,7 +248,8 @@ struct PrefillPlan {
   int subs, splits;
 };
 
-// Estimated us of a plan: the longest item's chain against the load per CU.
+// Estimated us of a plan, to choose the sets: the longest item's chain against
+// the load per CU.
 // More sets shorten the chain (0.84 / 0.57 / 0.50 us a tile of a lone workgroup
 // with 1 / 2 / 4 sets) at the price of a longer start per item and, with 4 (128
 // KB of LDS), no second workgroup beside it. Splits add the partials' traffic
@@ -280,25 +281,75 @@ double prefill_us(int64_t bh, int32_t q_len, int32_t kv_len, int subs, int split
   return walk + (partials > 0 ? c.merge + c.partial * mb : 0.0);
 }
 
-// The cheapest plan by that estimate; the plain kernel without splits unless
-// another is 5% cheaper. Splitting pays only for few items (at most 128 tried:
-// then a chain cannot be shortened by sets alone), and never with 4 sets. A
-// caller's own split count is taken. us, one set and the earlier split rule ->
-// plan, 12 heads: 1 x 3088 (4 splits) 39.8 -> 32.4 (4 sets), 1 x 4096 57.5 -> 41.6 (4), 2
-// x 2048 35.7 -> 28.0 (2), 4 x 1024 25.6 -> 18.3 (2), 8 x 512 (2 splits) 19.7 -> 12.9 (1),
-// 1 x 128 queries over 4096 keys 15 as before (1, 16 splits). Over the 100 shapes 11%
-// less time (geometric mean), 0.3% above the best plan of each.
+// The same to choose between splits and sets alone where the items are few: a
+// lone workgroup's chain carries 2-3 us of first loads and tail more than the fit
+// above gives it; partials cost by the rows really written; a merge beyond 8
+// splits takes a second round trip (1 us); and every further workgroup per CU is a
+// step, since the items are about as long as each other and end together (2 x 12
+// heads, 200 queries over 4296 keys, two sets: 5 splits = 240 workgroups 19.7 us, 6 =
+// 288 24.0). Fitted to 440 shapes, 3400 timings (65-4096 queries, 65-12000 keys, 12-512
+// heads in all; rms error 5%).
+double prefill_few_us(int64_t bh, int32_t q_len, int32_t kv_len, int subs, int splits) {
+  struct Cost {
+    double chain0, chain, load0, load, item;                // without partials
+    double split0, split_chain, split_load, step, partial;  // with
+  };
+  static constexpr Cost kCost[3] = {{4.4, 0.84, 0.0, 0.434, 2.28, 6.84, 0.814, 0.374, 1.27, 0.0205},
+                                    {5.47, 0.57, 0.0, 0.436, 3.55, 8.17, 0.546, 0.4735, 2.11, 0.0194},
+                                    {7.7, 0.477, 4.4, 0.56, 6.85}};  // 4 sets: never with splits
+  const Cost& c = kCost[subs >> 1];
+  const int split_tiles = ((kv_len + splits - 1) / splits + 63) / 64;
+  int longest = 0;
+  int64_t tiles = 0, items = 0, rows = 0;  // rows: of all partials
+  for (int q0 = 0; q0 < q_len; q0 += 128) {
+    const int t = (kv_len - q_len + std::min(q0 + 128, q_len) + 63) / 64;
+    const int n = splits == 1 ? 1 : (t + split_tiles - 1) / split_tiles;
+    longest = std::max(longest, std::min(t, split_tiles));
+    tiles += t;
+    items += n;
+    rows += n > 1 ? (int64_t)n * std::min(128, q_len - q0) : 0;
+  }
+  const double cu_tiles = (double)(tiles * bh) / 256.0, cu_items = (double)(items * bh) / 256.0;
+  if (rows > 0) {
+    const double chain = c.split0 + c.split_chain * longest, load = c.split_load * cu_tiles;
+    return std::sqrt(chain * chain + load * load) + c.step * (std::ceil(cu_items) - 1.0) +
+           c.partial * (double)(rows * bh) / 128.0 + (splits > 8 ? 1.0 : 0.0);
+  }
+  const double chain = c.chain0 + c.chain * longest, load = c.load0 + c.load * cu_tiles + c.item * cu_items;
+  return subs == 4 ? std::max(chain, load) : std::sqrt(chain * chain + load * load);
+}
+
+// The cheapest plan: of the sets without splits, one unless another is 5% cheaper;
+// then splits, with one or two sets, where they are 3% cheaper still. Splitting
+// pays only for few items (at most 128 tried: then a chain cannot be shortened by
+// sets alone) with at least as many keys before the queries as among them (with
+// fewer the items are too unequal), and never with 4 sets. A caller's own split
+// count is taken. us, one set and the earlier split rule -> plan, 12 heads: 1 x 3088 (4
+// splits) 39.8 -> 32.4 (4 sets), 1 x 4096 57.5 -> 41.6 (4), 2 x 2048 35.7 -> 28.0 (2), 4 x 1024
+// 25.6 -> 18.3 (2), 8 x 512 (2 splits) 19.7 -> 12.9 (1); 2 x 200 queries over 4296 keys (11
+// splits) 21.3 -> 19.7 (2 sets, 5 splits), 1 x 136 over 2849 (12) 15.8 -> 13.6 (2, 8), 1 x
+// 71 over 799 (4) 10.2 as before (two sets without splits: 13.0). Over those 440
+// shapes 8% less time (geometric mean), 0.7% above the best plan of each; 366 others 9%
+// less, five of them 3-8% slower than with the earlier rule (one set was better
+// where the estimates of one and two differ by less than they err).
 PrefillPlan prefill_plan(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len, int32_t n_splits,
                          bool automatic) {
   constexpr int64_t kSplitItems = 128;
   const int64_t bh = (int64_t)batch * heads;
-  const int first = automatic ? 1 : n_splits;
-  const int last = !automatic || bh * ((q_len + 127) / 128) <= kSplitItems ? n_splits : 1;
-  PrefillPlan best{1, first};
-  double cost = 0.95 * prefill_us(bh, q_len, kv_len, 1, first);
-  for (int splits = first; splits <= last; ++splits)
-    for (int subs = 1; subs <= (splits == 1 ? 4 : 2); subs *= 2) {
-      const double us = prefill_us(bh, q_len, kv_len, subs, splits);
+  PrefillPlan best{1, automatic ? 1 : n_splits};
+  double cost = 0.95 * prefill_us(bh, q_len, kv_len, 1, best.splits);
+  for (int subs = 2; subs <= (best.splits == 1 ? 4 : 2); subs *= 2) {
+    const double us = prefill_us(bh, q_len, kv_len, subs, best.splits);
+    if (us < cost) {
+      cost = us;
+      best.subs = subs;
+    }
+  }
+  if (!automatic || bh * ((q_len + 127) / 128) > kSplitItems || q_len > kv_len / 2) return best;
+  cost = 0.97 * prefill_few_us(bh, q_len, kv_len, best.subs, 1);
+  for (int splits = 2; splits <= n_splits; ++splits)
+    for (int subs = 1; subs <= 2; ++subs) {
+      const double us = prefill_few_us(bh, q_len, kv_len, subs, splits);
       if (us < cost) {
         cost = us;
         best = PrefillPlan{subs, splits};
@@ -342,6 +393,28 @@ int32_t decode_ranges(int64_t units, int32_t kv_len, int32_t n_splits, bool auto
   return automatic && kv_len - kv_len / s < 1000 ? 1 : s;
 }
 
+// What a decode call runs: sets per workgroup (prefill), key ranges and their
+// length. Ranges are whole 32-key chunks, the kernels' load and compute unit (a
+// range ending mid-chunk would load the chunk's other half twice); of prefill
+// whole 64-key tiles.
+struct DecodePlan {
+  int subs, splits, split_len;
+};
+
+DecodePlan decode_plan(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len, int32_t n_splits,
+                       bool automatic) {
+  PrefillPlan p{1, 1};
+  int unit = 32;
+  if (q_len < kPrefillMinQ) {
+    p.splits = decode_ranges((int64_t)batch * heads * decode_q_tiles(q_len), kv_len, n_splits, automatic);
+  } else {
+    p = prefill_plan(batch, heads, q_len, kv_len, n_splits, automatic);
+    unit = 64;
+  }
+  const int len = (kv_len + p.splits - 1) / p.splits;
+  return DecodePlan{p.subs, p.splits, (len + unit - 1) / unit * unit};
+}
+
 int run_decode(const void* q, const void* k, const void* v, void* o, int32_t batch,
                int32_t heads, int32_t q_len, int32_t kv_len, int32_t block_size,
                int32_t n_splits, bool automatic, const int64_t* strides, float scale, void* workspace,
@@ -353,8 +426,8 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
     return fail(BD3_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
   if (need > 0 && (workspace == nullptr || !aligned16(workspace)))
     return fail(BD3_EINVAL, "workspace must be a 16-byte aligned device pointer");
-  if (q_len < kPrefillMinQ)
-    n_splits = decode_ranges((int64_t)batch * heads * q_tiles, kv_len, n_splits, automatic);
+  const DecodePlan plan = decode_plan(batch, heads, q_len, kv_len, n_splits, automatic);
+  if (q_len < kPrefillMinQ) n_splits = plan.splits;
   bd3::DecodeArgs a;
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
@@ -374,26 +447,17 @@ int run_decode(const void* q, const void* k, const void* v, void* o, int32_t bat
   a.kv_len = kv_len;
   a.bs = block_size;
   a.n_splits = n_splits;
-  // Split length: ceil(kv_len / n_splits) rounded up to whole 32-key chunks
-  // (the kernels' load and compute unit; a split ending mid-chunk would load
-  // the chunk's other half twice).
-  int sl = (kv_len + n_splits - 1) / n_splits;
-  sl = (sl + 31) / 32 * 32;
-  a.split_len = sl;
-  a.subs = 1;
+  a.split_len = plan.split_len;
+  a.subs = plan.subs;
   a.q_tiles = q_tiles;
   a.scale_log2 = scale * bd3::kLog2e;
   if (q_len >= kPrefillMinQ) {
-    // 128-row tiles, splits of whole 64-key tiles; partials in the same
-    // layout (one slot per 32-row tile and split).
+    // 128-row tiles; partials in the same layout (one slot per 32-row tile and
+    // split).
     for (int i = 1; i <= 2; ++i) {
       const int st = check_dma_stride(strides + 3 * i, i == 1 ? "k" : "v");
       if (st) return st;
     }
-    const PrefillPlan plan = prefill_plan(batch, heads, q_len, kv_len, n_splits, automatic);
-    a.subs = plan.subs;
-    int pl = (kv_len + plan.splits - 1) / plan.splits;
-    a.split_len = (pl + 63) / 64 * 64;
     return hip_status(bd3::launch_prefill(a, static_cast<hipStream_t>(stream)), "prefill launch");
   }
   return hip_status(bd3::launch_decode(a, kDecodeQT, static_cast<hipStream_t>(stream)), "decode launch");
@@ -649,6 +713,15 @@ int bd3_attn_bwd_noalloc(const void* q, const void* k, const void* v, const void
 int32_t bd3_decode_auto_splits(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len) {
   if (batch < 1 || heads < 1 || q_len < 1 || kv_len < 1) return 1;
   return auto_splits(batch, heads, q_len, kv_len);
+}
+
+int32_t bd3_decode_ranges(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len, int32_t n_splits) {
+  if (batch < 1 || heads < 1 || q_len < 1 || kv_len < 1 || q_len > kv_len || n_splits < 0 || n_splits > kv_len)
+    return 1;
+  const bool automatic = n_splits == 0;
+  if (automatic) n_splits = auto_splits(batch, heads, q_len, kv_len);
+  const DecodePlan p = decode_plan(batch, heads, q_len, kv_len, n_splits, automatic);
+  return (kv_len + p.split_len - 1) / p.split_len;
 }
 
 size_t bd3_decode_workspace_bytes(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len,

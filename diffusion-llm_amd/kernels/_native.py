@@ -52,6 +52,7 @@ SIGNATURES: dict[str, tuple] = {
     "bd3_decode": (ctypes.c_int, [_c_p, _c_p, _c_p, _c_p, _i32, _i32, _i32, _i32, _i32, _i32,
                                   _i64p, _f32, _c_p, _sz, _c_p]),
     "bd3_decode_auto_splits": (_i32, [_i32, _i32, _i32, _i32]),
+    "bd3_decode_ranges": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "bd3_decode_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "bd3_decode_splitkv": (ctypes.c_int, [_c_p, _c_p, _c_p, _c_p, _i32, _i32, _i32, _i32, _i32, _i32,
                                           _i32, _i64p, _f32, _c_p, _sz, _c_p]),

@@ -232,6 +232,15 @@ int32_t bd3_decode_auto_splits(int32_t batch, int32_t heads, int32_t q_len,
                                int32_t kv_len);
 
 /*
+ * Ranges that a call really cuts the keys into: bd3_decode for n_splits 0,
+ * bd3_decode_splitkv for others (q_len <= 64: at most 256 workgroups are cut
+ * for, and ranges are whole 32-key chunks; q_len > 64: whole 64-key tiles). 1:
+ * no partials and no merge. Host only. No reference counterpart.
+ */
+int32_t bd3_decode_ranges(int32_t batch, int32_t heads, int32_t q_len,
+                          int32_t kv_len, int32_t n_splits);
+
+/*
  * Workspace bytes for a split-KV decode with n_splits splits (0 = the auto
  * count bd3_decode uses):
  * fp32 partial O and LSE per (batch*head, query tile, split). 0 when a

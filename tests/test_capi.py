@@ -330,6 +330,29 @@ def test_workspace_sizes(lib):
         32, 12, 16, 4112, 64, s)
 
 
+def test_prefill_ranges(lib):
+    """Ranges a call of more than 64 queries cuts its keys into. Automatic: few
+    items with long chains are split (one chain of 13 tiles takes longer than
+    4 ranges and their merge; 48 row tiles in 5 ranges give each CU at most
+    one workgroup), items that sets of waves shorten enough are not, nor are
+    queries without as many keys before them; never more than the workspace
+    is sized for. A caller's own count is taken, in whole 64-key tiles."""
+    auto = lambda *shape: lib.bd3_decode_ranges(*shape, 0)
+    assert [auto(*s) for s in ((1, 12, 71, 799), (3, 12, 92, 775), (1, 12, 88, 714), (1, 16, 423, 1265))] == [4, 4, 3, 4]
+    assert auto(2, 12, 200, 4296) == 5 and auto(1, 12, 128, 4096) == 8
+    for s in ((1, 12, 3088, 3088), (2, 12, 2048, 2048), (8, 12, 512, 512), (32, 12, 128, 4112), (1, 12, 1064, 1064)):
+        assert auto(*s) == 1, s
+    for B in (1, 3, 8):
+        for q in (65, 128, 200, 700, 2048):
+            for kv in (q, q + 100, 3 * q, q + 5000):
+                assert 1 <= auto(B, 12, q, kv) <= lib.bd3_decode_auto_splits(B, 12, q, kv)
+                for n in (1, 2, 5, 16):
+                    if n <= kv:
+                        length = -(-(-(-kv // n)) // 64) * 64
+                        assert lib.bd3_decode_ranges(B, 12, q, kv, n) == -(-kv // length)
+    assert lib.bd3_decode_ranges(1, 12, 128, 100, 0) == lib.bd3_decode_ranges(0, 12, 128, 200, 0) == 1
+
+
 def test_qkv_rope_validation(lib):
     xs = _i64([32 * 2304, 2304])
     os_ = _i64([12 * 32 * 64, 32 * 64, 64] * 3)

@@ -311,7 +311,8 @@ def test_decode_routes_match_oracle(cuda, record_error, B, H, q_len, kv_len, bs,
 # a ragged last row tile and last key tile, masks per strip and per element;
 # with one split, with splits that keep two sets, and the library's choice.
 WAVE_SETS = [(1, 1, 65, 5000, 16, 1), (1, 1, 129, 5300, 64, 1), (1, 1, 5200, 5200, 5, 1), (1, 2, 4000, 4000, 4, 1),
-             (1, 1, 1000, 1000, 16, 1), (2, 1, 200, 300, 3, 1), (1, 1, 300, 1400, 16, 2), (1, 12, 1600, 3001, 16, 1)]
+             (1, 1, 1000, 1000, 16, 1), (2, 1, 200, 300, 3, 1), (1, 1, 300, 1400, 16, 2), (1, 12, 1600, 3001, 16, 1),
+             (1, 12, 71, 799, 16, 4), (2, 12, 200, 4296, 16, 5), (1, 12, 128, 4096, 32, 16)]
 
 
 @pytest.mark.gpu
