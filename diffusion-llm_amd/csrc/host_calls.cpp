@@ -122,8 +122,8 @@ struct Args {
     if (v < INT32_MIN || v > INT32_MAX) throw Refused{PyExc_OverflowError, "argument does not fit 32 bits"};
     return (int32_t)v;
   }
-  uint64_t unsigned64() {
-    const unsigned long long v = PyLong_AsUnsignedLongLong(a[at++]);
+  uint64_t unsigned64() {  // modulo 2^64, any integer, as ctypes takes it (a seed or counter set by the caller)
+    const unsigned long long v = PyLong_AsUnsignedLongLongMask(a[at++]);
     if (v == (unsigned long long)-1 && PyErr_Occurred()) throw python_error();
     return v;
   }

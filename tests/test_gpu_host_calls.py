@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import threading
 
+import numpy as np
 import pytest
 import torch
 
@@ -55,6 +56,19 @@ def test_operands_off_the_gpu_are_refused_without_one():
     ):
         with pytest.raises(AssertionError, match="CUDA"):
             call()
+
+
+def test_seeds_are_taken_modulo_2_64():
+    """A generator whose seed or offset was set by hand to a negative, large or
+    numpy integer is accepted, as it was by ctypes (the call gets as far as the
+    refusal of its CPU tensors)."""
+    host = _native.host()
+    x, block = torch.zeros(1, 2, 64), torch.zeros(1, 2, dtype=torch.int64)
+    for seed, offset in ((-1, 0), (1 << 64, -5), (np.int64(-7), np.uint64(1 << 63))):
+        with pytest.raises(AssertionError, match="CUDA"):
+            host.subs_sample(x, block, 63, 0.5, None, seed, offset)
+    with pytest.raises(TypeError):
+        host.subs_sample(x, block, 63, 0.5, None, 1.5, 0)
 
 
 def rnd(dev, *shape, seed=0, dtype=BF):
@@ -161,6 +175,17 @@ def test_one_operand_off_the_gpu_is_refused(cuda):
                 (q, q[:, :, :128], q, q, lse, q), (q.half(), q, q, q, lse, q), (q, q, q, q, lse, q[:, :, :128])):
         with pytest.raises(AssertionError):
             train(*bad)
+
+
+@pytest.mark.gpu
+def test_negative_seed_is_its_value_modulo_2_64(cuda):
+    logits, block = rnd(cuda, 8, 3000, seed=9), torch.full((8,), 2999, device=cuda)
+    outs = []
+    for seed, offset in ((-3, -2), ((1 << 64) - 3, (1 << 64) - 2)):
+        g = PhiloxStream(0)
+        g.seed, g.offset = seed, offset
+        outs.append(subs_sample_step(logits, block, 2999, 0.1, generator=g))
+    assert torch.equal(*outs)
 
 
 @pytest.mark.gpu
