@@ -85,7 +85,8 @@ _lock = threading.Lock()
 
 
 def lib() -> ctypes.CDLL:
-    """Load libbd3attn.so once; raise RuntimeError if it was not built."""
+    """Load libbd3attn.so once; raise RuntimeError if it was not built, or
+    from other sources (BD3ATTN_LIB names any file)."""
     global _lib
     if _lib is None:
         with _lock:
@@ -96,6 +97,11 @@ def lib() -> ctypes.CDLL:
                         "`python -c 'import __graft_entry__ as g; g.build()'` "
                         "(or python diffusion-llm_amd/csrc/build.py)")
                 handle = ctypes.CDLL(str(LIB_PATH))
+                missing = [name for name in SIGNATURES if not hasattr(handle, name)]
+                if missing:
+                    raise RuntimeError(
+                        f"{LIB_PATH} is not the library of this package's version (no {', '.join(missing)}): "
+                        "build it again with `python -c 'import __graft_entry__ as g; g.build()'`")
                 for name, (res, args) in SIGNATURES.items():
                     fn = getattr(handle, name)
                     fn.restype = res

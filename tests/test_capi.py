@@ -41,6 +41,16 @@ def test_abi_version(lib):
     assert lib.bd3_abi_version() == 2
 
 
+def test_library_of_other_sources_is_named(lib, monkeypatch):
+    """A shared library without this package's symbols (an older build named
+    by BD3ATTN_LIB) is refused with its path and what it lacks."""
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "LIB_PATH", _native.HOST_PATH)
+    with pytest.raises(RuntimeError, match=r"bd3_host\.so is not the library.*bd3_subs_sample_ws"):
+        _native.lib()
+    assert _native._lib is None
+
+
 @pytest.mark.parametrize("n,bs", [(128, 1), (128, 16), (256, 4), (256, 100), (384, 64), (512, 512),
                                   (1024, 16), (2048, 256)])
 def test_census_matches_oracle(lib, n, bs):
