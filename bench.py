@@ -370,28 +370,28 @@ def decode_bench(device, reps: int):
                                        n_splits, st, 1.0 / 8, ptr(ws), nbytes, stream))
         return call
 
-    # At this shape (384 batch*heads) 2 or 3 splits write fp32 partials to HBM
-    # and merge them in a second launch (the reference's split_kv_kern +
-    # split_kv_reduce_kern); from 4 splits on one workgroup per head takes all
-    # of its splits and merges them on chip.
+    # `n_splits` is what the call asks for, `ranges` what the library cuts: at
+    # this shape (384 batch*heads, more than the 256 CUs) every count runs as one
+    # range per head, without partials or a merge.
     for ns in (1, 2, 3, 4, 8, 16, 0):
         eff = ns if ns else -(-kv_len // 256)  # 0: the reference's SPLIT_N = 256 rule
         t = bench(run(eff), warmup=5, rep=reps, flush=True)
-        merge = "none" if eff == 1 else ("partials in HBM + merge launch" if eff < 4 else "on chip, per head")
-        rows.append({"n_splits": eff, "rule": "reference ceil(kv/256)" if ns == 0 else "explicit",
+        ranges = L.bd3_decode_ranges(B, H, q_len, kv_len, eff)
+        merge = "none" if ranges == 1 else "partials in HBM + merge launch"
+        rows.append({"n_splits": eff, "ranges": ranges, "rule": "reference ceil(kv/256)" if ns == 0 else "explicit",
                      "merge": merge, "us": t.mean_ms * 1e3, "us_median": t.median_ms * 1e3,
                      "us_p20": t.p20_ms * 1e3, "us_p80": t.p80_ms * 1e3,
                      "GB_s": kv_bytes / (t.mean_ms * 1e-3) / 1e9})
     # the library's auto split (bd3_decode)
     nb_auto = L.bd3_decode_workspace_bytes(B, H, q_len, kv_len, D, 0)
     ws_auto = torch.empty(max(nb_auto, 1), device=device, dtype=torch.uint8)
-    auto_splits = L.bd3_decode_auto_splits(B, H, q_len, kv_len)
+    auto_ranges = L.bd3_decode_ranges(B, H, q_len, kv_len, 0)
 
     def call_auto():
         check(L.bd3_decode(ptr(q), ptr(k), ptr(v), ptr(o), B, H, q_len, kv_len, D, bs, st, 1.0 / 8,
                            ptr(ws_auto), nb_auto, stream))
     t = bench(call_auto, warmup=5, rep=reps, flush=True)
-    rows.append({"n_splits": auto_splits, "rule": "auto (bd3_decode)", "us": t.mean_ms * 1e3,
+    rows.append({"n_splits": auto_ranges, "ranges": auto_ranges, "rule": "auto (bd3_decode)", "us": t.mean_ms * 1e3,
                  "us_median": t.median_ms * 1e3, "us_p20": t.p20_ms * 1e3, "us_p80": t.p80_ms * 1e3,
                  "GB_s": kv_bytes / (t.mean_ms * 1e-3) / 1e9})
     best = max(rows, key=lambda r: r["GB_s"])
@@ -413,7 +413,8 @@ def decode_b1_bench(device, reps: int):
     (the reference rule: ceil(kv_len / 256) splits, prefill falls back to
     bsdfa as the reference does, kernels/SplitKVDecodeAttention.py:140-147).
     HIP events, 1 GiB cache eviction before each call; KV-read GB/s counts the
-    K and V bytes the rows can see."""
+    K and V bytes the rows can see; n_splits is the number of key ranges that
+    run."""
     import torch
     from kernels.BlockSparseDecodeAttention import block_sparse_decode_attention
     from kernels.SplitKVDecodeAttention import split_kv_decode_attention
@@ -425,8 +426,10 @@ def decode_b1_bench(device, reps: int):
         k, v = seeded_bf16((1, 12, kv_len, D), 4, 2, device)
         kv_bytes = 2 * 12 * kv_len * D * 2
         for name, fn, splits in (
-                ("bsdfa", block_sparse_decode_attention, lib().bd3_decode_auto_splits(1, 12, q_len, kv_len)),
-                ("split_kv", split_kv_decode_attention, -(-kv_len // 256) if q_len <= 64 else "bsdfa fallback")):
+                ("bsdfa", block_sparse_decode_attention, lib().bd3_decode_ranges(1, 12, q_len, kv_len, 0)),
+                ("split_kv", split_kv_decode_attention,
+                 lib().bd3_decode_ranges(1, 12, q_len, kv_len, -(-kv_len // 256)) if q_len <= 64
+                 else "bsdfa fallback")):
             t = bench(lambda: fn(q, k, v, 16), warmup=5, rep=reps, flush=True)
             out[f"{shape}_{name}"] = {"q_len": q_len, "kv_len": kv_len, "heads": 12, "n_splits": splits,
                                       "us": t.median_ms * 1e3, "us_p20": t.p20_ms * 1e3, "us_p80": t.p80_ms * 1e3,
@@ -786,7 +789,7 @@ def main(argv=None) -> int:
     if not args.no_decode:
         result["decode"] = decode_bench(device, reps=30)
         for r in result["decode"]["rows"]:
-            log(f"decode n_splits={r['n_splits']:3d} ({r['rule']}, merge {r.get('merge', 'none')}): "
+            log(f"decode n_splits={r['n_splits']:3d} ({r['rule']}, {r['ranges']} ranges, merge {r.get('merge', 'none')}): "
                 f"{r['us']:.1f} us, {r['GB_s']:.0f} GB/s")
     if not args.no_decode:
         result["decode_batch1"] = decode_b1_bench(device, reps=30)

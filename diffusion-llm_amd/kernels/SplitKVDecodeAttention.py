@@ -3,9 +3,12 @@
 Drop-in for the reference's kernels/SplitKVDecodeAttention.py:
 `split_kv_decode_attention(q, k, v, block_size)` gives the same result as
 block_sparse_decode_attention with the keys split across workgroups; each
-split writes a normalised fp32 partial and its LSE, merged with LSE weights.
-Adds an optional `n_splits` (default: the reference rule
-ceil(kv_len / SPLIT_N), :147). Runs bd3_decode_splitkv in libbd3attn.so.
+range of keys writes a normalised fp32 partial and its LSE, merged with LSE
+weights. Adds an optional `n_splits` (default: the reference rule
+ceil(kv_len / SPLIT_N), :147): the most ranges the keys are cut into. Up to 64
+queries are cut into no more than fill the GPU (256 workgroups over all
+sequences, heads and query tiles), the call's result being the same;
+bd3_decode_ranges tells the number. Runs bd3_decode_splitkv in libbd3attn.so.
 """
 import torch
 from torch import Tensor
@@ -25,8 +28,8 @@ def split_kv_decode_attention(
     n_splits: int | None = None,
 ) -> Tensor:
     """Same result as block_sparse_decode_attention, with the keys split
-    across workgroups so a decode step fills the GPU
-    (reference: kernels/SplitKVDecodeAttention.py:130-171)."""
+    across workgroups so a decode step fills the GPU, into at most n_splits
+    ranges (reference: kernels/SplitKVDecodeAttention.py:130-171)."""
     kv_len = k.shape[2]
     if q.shape[2] > 64 and n_splits is None:
         # prefill: many query tiles already fill the GPU (reference :140-142)

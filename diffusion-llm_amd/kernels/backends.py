@@ -16,7 +16,7 @@ visibility rule from the block size and the layout it serves.
     name      layout of (q, k, v)                         rule
     bsfa      training sequence cat(x_t, x_0), length 2n  BD3-LM mask; fwd + bwd
     bsdfa     q = last q_len of the kv_len positions      block-causal; fwd only
-    split_kv  as bsdfa                                    as bsdfa, keys cut into
+    split_kv  as bsdfa                                    as bsdfa, keys cut into at most
                                                           the reference's 256-key splits
 """
 from __future__ import annotations
@@ -56,8 +56,8 @@ def bsdfa(q, k, v, mask=None, block_size=None):
 
 
 def split_kv(q, k, v, mask=None, block_size=None):
-    """Same result as bsdfa, with the keys cut into ceil(kv_len / 256) splits
-    merged by their log-sum-exp (bd3_decode_splitkv)."""
+    """Same result as bsdfa, with the keys cut into up to ceil(kv_len / 256)
+    ranges merged by their log-sum-exp (bd3_decode_splitkv)."""
     return torch.ops.bd3.decode(q, k, v, block_size, _REFERENCE_SPLITS)
 
 

@@ -11,8 +11,8 @@ carries its backward (register_autograd).
     torch.ops.bd3.attn_bwd(q, k, v, O, L, dO, block_size) -> (dQ, dK, dV)
     torch.ops.bd3.decode(q, k, v, block_size, n_splits, token_major=False) -> O
         n_splits 0: the library's automatic split (bd3_decode), -1: the reference's split
-        rule (ceil(kv_len / 256), split_kv_decode_attention's default), > 0: that many
-        splits; token_major: O is a view of (batch, q_len, heads, head_dim) memory
+        rule (ceil(kv_len / 256), split_kv_decode_attention's default), > 0: at most that
+        many (split_kv_decode_attention); token_major: O is a view of (batch, q_len, heads, head_dim) memory
 """
 from __future__ import annotations
 

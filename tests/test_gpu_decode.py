@@ -50,9 +50,9 @@ def test_splitkv_matches_oracle(cuda, B, H, q_len, kv_len, bs, n_splits):
     assert max_abs(o, ref) <= OUT_TOL
 
 
-# Shapes where one workgroup takes several consecutive splits (batch * heads * n_splits > 512 and
-# at least 4 splits per workgroup): ragged key counts, short or empty last splits, q_len 1..16,
-# block sizes off the 16-key strips.
+# More splits asked for than fill the GPU (batch * heads * n_splits > 512): the keys are cut into
+# fewer ranges, one where there are 128 heads or more. Ragged key counts, q_len 1..16, block sizes
+# off the 16-key strips.
 GROUPED = [(4, 12, 16, 1000, 16, 33), (8, 12, 7, 3001, 5, 20), (2, 16, 16, 4112, 16, 64),
            (16, 12, 1, 777, 16, 12), (8, 8, 16, 2048, 64, 40), (3, 12, 11, 1234, 3, 30)]
 
@@ -60,9 +60,9 @@ GROUPED = [(4, 12, 16, 1000, 16, 33), (8, 12, 7, 3001, 5, 20), (2, 16, 16, 4112,
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,q_len,kv_len,bs,n_splits", GROUPED)
 def test_grouped_splits_match_oracle(cuda, record_error, B, H, q_len, kv_len, bs, n_splits):
-    """decode16_partial with several splits per workgroup (each wave's share of
-    a split merged on chip, heads starting at rotated splits) against the
-    oracle and against one split."""
+    """decode16_partial asked for more splits than it takes (5, 2, 8, 1, 4 and
+    7 ranges) against the oracle and against one split."""
+    assert 1 <= lib().bd3_decode_ranges(B, H, q_len, kv_len, n_splits) <= max(1, 256 // (B * H)) < n_splits
     q, k, v = decode_inputs(B, H, q_len, kv_len, seed=B * 1000 + kv_len + n_splits)
     qd, kd, vd = (t.to(cuda, torch.bfloat16) for t in (q, k, v))
     o = splitkv_capi(qd, kd, vd, bs, n_splits)
@@ -79,7 +79,9 @@ def test_grouped_splits_match_oracle(cuda, record_error, B, H, q_len, kv_len, bs
 def test_config3_split_invariance(cuda):
     """32 sequences x 12 heads, 16 queries over a
     4096 + 16 cache; splits {1, 4, 8, 16} and the reference default rule
-    all match the oracle and each other."""
+    all match the oracle and each other. 384 heads fill the GPU, so every
+    count runs as one range (the same launch); the first sequence alone (12
+    heads) runs the counts themselves."""
     B, H, q_len, kv_len, bs = 32, 12, 16, 4112, 16
     q, k, v = decode_inputs(B, H, q_len, kv_len, seed=0)
     qd, kd, vd = (t.to(cuda, torch.bfloat16) for t in (q, k, v))
@@ -92,6 +94,13 @@ def test_config3_split_invariance(cuda):
         assert max_abs(o, ref) <= OUT_TOL
     for o in outs[1:]:
         assert max_abs(o, outs[0]) <= 1e-2
+    counts = (1, 4, 8, 16)
+    assert [lib().bd3_decode_ranges(B, H, q_len, kv_len, s) for s in counts] == [1, 1, 1, 1]
+    assert [lib().bd3_decode_ranges(1, H, q_len, kv_len, s) for s in counts] == [1, 4, 8, 15]  # 288 keys each
+    one = [splitkv_capi(qd[:1], kd[:1], vd[:1], bs, s) for s in counts]
+    torch.cuda.synchronize()
+    for o in one:
+        assert max_abs(o, ref[:1]) <= OUT_TOL and max_abs(o, one[0]) <= 1e-2
 
 
 # q_len > 64 runs the prefill kernel: 128-row query tiles, splits of whole
@@ -195,9 +204,10 @@ def test_batch1_profiling_shapes(cuda, record_error, shape, backend):
 @pytest.mark.gpu
 def test_cached_step_every_split_count(cuda, record_error):
     """The reference's batch-1 cached shape at every split count 1-32 (one
-    partial per split, merged by decode_combine: 7-14 splits of 256-512 keys,
-    ragged last splits, 17-32 splits through the 32-split merge) against the
-    oracle; then 512 and 513 heads at two splits (q_len 9, block 7)."""
+    partial per range, merged by decode_combine: 7-14 ranges of 256-512 keys,
+    ragged last ranges, 17-21 through the 32-range merge, which 22-32 take
+    as well: 12 heads are cut into at most 21) against the oracle; then 512 and
+    513 heads at two splits (q_len 9, block 7), which run as one."""
     q, k, v = decode_inputs(1, 12, 16, 3584, seed=11)
     ref = decode_attention(q, k, v, 16)
     qd, kd, vd = (t.to(cuda, torch.bfloat16) for t in (q, k, v))
@@ -212,6 +222,24 @@ def test_cached_step_every_split_count(cuda, record_error):
         o = splitkv_capi(*(t.to(cuda, torch.bfloat16) for t in (q, k, v)), 7, 2)
         torch.cuda.synchronize()
         record_error(f"decode O max-abs ({B * H} heads)", max_abs(o, decode_attention(q, k, v, 7)), OUT_TOL)
+
+
+# The merges no other test reaches: 32 workgroups in one round trip, more in groups
+# of 8 (33, 36, 40, 64, 85 and 256 of them: a last group of one to eight), for both
+# kernels; the last of them short, or with no keys left (19, 29 of 33, 58 of 85).
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,q_len,kv_len,bs,n_splits,ranges",
+                         [(1, 8, 16, 3000, 16, 32, 32), (1, 7, 16, 1200, 16, 33, 19), (1, 7, 16, 4500, 5, 33, 29),
+                          (1, 7, 5, 1152, 16, 50, 36), (2, 3, 16, 5000, 4, 40, 40), (1, 4, 16, 2048, 16, 64, 64),
+                          (1, 1, 1, 8192, 16, 300, 256), (3, 1, 16, 5500, 7, 100, 58), (1, 3, 32, 5440, 32, 90, 85),
+                          (2, 1, 33, 2080, 16, 40, 33)])
+def test_every_merge_of_ranges(cuda, record_error, B, H, q_len, kv_len, bs, n_splits, ranges):
+    print(f"merge of {ranges} ranges B={B} H={H} q_len={q_len} kv_len={kv_len}", flush=True)
+    assert lib().bd3_decode_ranges(B, H, q_len, kv_len, n_splits) == ranges
+    q, k, v = decode_inputs(B, H, q_len, kv_len, seed=kv_len + n_splits)
+    o = splitkv_capi(*(t.to(cuda, torch.bfloat16) for t in (q, k, v)), bs, n_splits)
+    torch.cuda.synchronize()
+    record_error("decode O max-abs (merge)", max_abs(o, decode_attention(q, k, v, bs)), OUT_TOL)
 
 
 @pytest.mark.gpu
