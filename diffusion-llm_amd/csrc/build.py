@@ -29,7 +29,7 @@ OBJ_DIR = PKG / "_build"
 ARCH = "gfx950"
 
 # -packed-fp32-ops: hipcc would otherwise fuse float pairs into
-# v_pk_{add,mul,fma}_f32, some forms of which are unreliable on this pool.
+# v_pk_{add,mul,fma}_f32, some forms of which have given wrong results on gfx950.
 # The host pass warns that it does not know the feature; that is harmless.
 # -mno-amdgpu-ieee -fno-honor-nans: the kernels never produce or consume
 # NaN (masked scores are -inf, every row has a live key), so the IEEE-mode

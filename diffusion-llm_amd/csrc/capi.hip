@@ -130,22 +130,21 @@ bd3::BwdArgs bwd_args(const void* q, const void* k, const void* v, const void* o
   return a;
 }
 
-// Sets of four waves per workgroup of the training launches: two where a few
-// long items leave the chip idle (the sets take an item's tiles in turn and add
-// up at its end), one where the launch is bound by its work. Both rules weigh
-// the longest item's chain against the load per workgroup slot; a two-set
-// workgroup's chain is 1.25-1.45 times shorter, but fewer of them fit (backward
-// 256 for 768, forward 512 of twice the waves for 1024) and each start-up is
-// longer. Fitted to 33 shapes, 12 heads a sequence, block 16, us with one -> two:
+// Sets of four waves per workgroup of the training launches (bwd_subs, fwd_subs):
+// two where a few long items leave the chip idle (the sets take an item's tiles
+// in turn and add up at its end), one where the launch is bound by its work. Both
+// rules weigh the longest item's chain against the load per workgroup slot; a
+// two-set workgroup's chain is 1.25-1.45 times shorter, but fewer of them fit
+// (backward 256 for 768, forward 512 of twice the waves for 1024) and each start-up
+// is longer. Fitted to 33 shapes, 12 heads a sequence, block 16, us with one -> two:
 // backward main launch 1 x n 256 14.9 -> 13.4, 1 x 1024 47.0 -> 35.5, 1 x 2048 94.5
 // -> 66.8, 1 x 3072 156.6 -> 129.4, 2 x 1024 51.4 -> 42.4, 3 x 512 28.0 -> 24.7; not 4 x
 // 512 32.8 (33.6), 3 x 1024 57.6 (59.1), 2 x 2048 116.5 (121.8), 8 x 256 19.9 (26.2),
 // 8 x 1024 115 (149). Forward 1 x 1024 18.5 -> 15.5, 1 x 2048 33.9 -> 28.4, 2 x 1024
 // 20.2 -> 18.8, 1 x 4096 76.8 -> 72.9; not 8 x 256 10.7 (11.3), 3 x 1024 23.1 (23.0), 6
-// x 512 16.5 (18.3), 8 x 1024 41.6 (47.1).
-
-// longest, total: cost units of the longest item and of all of them (3 a tile for
-// a dQ item, 4 for a dK/dV item); items of all batch*heads. Times in us.
+// x 512 16.5 (18.3), 8 x 1024 41.6 (47.1). bwd_subs takes cost units: of the longest
+// item and of all of them (3 a tile for a dQ item, 4 for a dK/dV item), and the items
+// of all batch*heads; its estimates are us.
 int bwd_subs(int longest, int64_t total, int64_t items) {
   const double load = (double)total / 768.0;
   const double chain1 = 5.0 + 0.33 * longest, work1 = 5.0 + 0.68 * load + 8.1 * (double)items / 768.0;
@@ -213,8 +212,9 @@ void bwd_order(bd3::BwdArgs& a, bool dq, bool dkdv) {
 constexpr int kPrefillMinQ = 65;
 
 // The most splits of an automatic prefill call, which sizes its workspace
-// (prefill_plan below takes fewer where that is faster): none when the (row tile, batch*head) items
-// alone fill half of the GPU's workgroup slots (4 per CU on 256 CUs);
+// (prefill_plan below takes fewer where that is faster): none when the (row
+// tile, batch*head) items alone fill half of the GPU's workgroup slots (4 per CU
+// on 256 CUs);
 // otherwise as few as keep the longest item (one split of one 128-row tile)
 // under the grid's total work spread over those slots, with kLoneTile = the
 // cost of a 64-key tile in a workgroup running alone on its CU relative to
@@ -837,8 +837,8 @@ namespace {
 
 // Slices a row of the sampling scan may be cut into (1: one workgroup per
 // row): each takes at least 2048 of the row's elements (one pair per thread),
-// and 16 of them put 16 rows on every CU; 24 measured the same (17.2 us a call
-// for one 16-token block). Above kSubsSpreadRows rows there is a workgroup for
+// and 16 of them put 16 rows on every CU (8, 16 and 24 take 12.5, 12.3 and 14.9
+// us a call for one 16-token block). Above kSubsSpreadRows rows there is a workgroup for
 // every CU four times over without slices.
 constexpr int kSubsSpread = 512;  // workgroups of a spread call: two 1024-thread ones per CU
 int subs_slices(int32_t rows, int32_t vocab) {

@@ -67,8 +67,6 @@ __device__ __forceinline__ void unpack8(const Raw8& r, int fp32, float (&v)[8]) 
   for (int e = 0; e < 8; ++e) v[e] = fp32 ? f[e] : b[e];
 }
 
-__device__ __forceinline__ void load8(const void* p, int fp32, float (&v)[8]) { unpack8(ld_raw8(p, fp32), fp32, v); }
-
 __device__ __forceinline__ void store8(void* p, int fp32, const float (&v)[8]) {
   if (fp32) {
     *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
@@ -121,15 +119,15 @@ __device__ __forceinline__ void store4(void* p, bool fp32, const float (&v)[4]) 
 // x + gate * y (gate_residual_kernel's dtypes and roundings), which is stored
 // too: one launch and one read of the residual instead of two of each
 // (DiTBlock.forward, model/modules.py:560-566 then the next sublayer's
-// :537-568). out_x may alias x (a wave has read its row before it writes it,
-// and no other wave reads it).
+// :537-568). out_x may alias x (a wave has read its chunks of the row before it
+// writes them, and no other wave uses them).
 //
 // A wave owns `a.wave_rows` consecutive rows; lane l holds the 4-element chunks
 // l, l + 64, ... of a row, so every load and store of a wave is one contiguous
-// piece. CH: chunks per lane. Rows of up to 4 chunks per
-// lane keep the gain, 1 + scale and shift (and the gate) in registers from row
-// to row and request the next row before they work on the current one; longer
-// rows load them per row. XF / MF / YF: x, the vectors, y in fp32.
+// piece. CH: chunks per lane. Rows of up to 4 chunks per lane keep the gain, 1 +
+// scale and shift (and the gate) in registers from row to row and request the
+// next row before they work on the current one; longer rows load them per row.
+// XF / MF / YF: x, the vectors, y in fp32.
 //
 // PAIR: rows of more than 2048, two waves (a 128-thread workgroup) to a row,
 // each with every other run of 64 chunks, and the sums exchanged through LDS:
@@ -340,23 +338,6 @@ __global__ __launch_bounds__(PAIR ? 128 : 256) void ln_modulate_kernel(GlueArgs 
   }
 }
 
-// 4 consecutive elements at p: fp32 (16 bytes) or bf16 (8 bytes), the dtype
-// fixed at compile time.
-template <bool F32>
-__device__ __forceinline__ void load4(const void* p, float (&v)[4]) {
-  if constexpr (F32) {
-    const f32x4 t = *reinterpret_cast<const f32x4*>(p);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = t[k];
-  } else {
-    const uint2 t = *reinterpret_cast<const uint2*>(p);
-    v[0] = __uint_as_float(t.x << 16);
-    v[1] = __uint_as_float(t.x & 0xffff0000u);
-    v[2] = __uint_as_float(t.y << 16);
-    v[3] = __uint_as_float(t.y & 0xffff0000u);
-  }
-}
-
 // x + gate * y with an fp32 residual (the result is fp32): 4 elements per
 // thread, so each load of x (16 bytes per lane) covers one contiguous 1 KB
 // per wave, where 8-element chunks (two 16-byte halves 32 bytes apart per
@@ -370,10 +351,16 @@ __global__ __launch_bounds__(256) void gate_residual_f32_kernel(GlueArgs a) {
   if (e >= (int64_t)a.rows * nch) return;
   const int row = (int)(e / nch), c = (int)(e - (int64_t)row * nch);
   const int b = row / a.seq, s = row - b * a.seq;
+  Raw4<true> xr;
+  Raw4<GF> gr;
+  Raw4<YF> yr;
+  xr.load(static_cast<const float*>(a.x) + (int64_t)b * a.sx_b + (int64_t)s * a.sx_s + 4 * c);
+  gr.load(elem(a.shift, GF, (int64_t)b * a.sm_b + 4 * c));  // gate
+  yr.load(elem(a.y, YF, (int64_t)b * a.sy_b + (int64_t)s * a.sy_s + 4 * c));
   float x[4], g[4], y[4];
-  load4<true>(static_cast<const float*>(a.x) + (int64_t)b * a.sx_b + (int64_t)s * a.sx_s + 4 * c, x);
-  load4<GF>(elem(a.shift, GF, (int64_t)b * a.sm_b + 4 * c), g);  // gate
-  load4<YF>(elem(a.y, YF, (int64_t)b * a.sy_b + (int64_t)s * a.sy_s + 4 * c), y);
+  xr.get(x);
+  gr.get(g);
+  yr.get(y);
   const bool gy_bf16 = !GF && !YF;
   f32x4 o;
 #pragma unroll

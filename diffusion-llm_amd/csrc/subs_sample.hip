@@ -40,8 +40,9 @@
 // pair about half of them), not by reading the logits. Against one 1024-thread
 // workgroup per row with three passes over an LDS copy of it (131 KB, so one
 // per CU) and the float64 path inside the last pass, per call at 50258 bf16
-// logits: 16 masked rows 56 -> 17 us (scan 7.5, finish 3.6), 256 rows half of
-// them masked 58.7 -> 20.1, all masked 58.7 -> 27.0. 1024 workgroups instead of
+// logits: 16 masked rows 57 -> 12.3 us (scan 7.7, finish 3.8), 256 rows half of
+// them masked 58.7 -> 20.1, all masked 58.7 -> 27.0; a block with no masked row
+// left 3-4 -> 5 us (the second launch: the host does not know the tokens). 1024 workgroups instead of
 // 512 take 26.4 and 32.3 us for the last two (every slice reads its whole row
 // for the maximum), 256 take 21.6 and 28.4; a slice per workgroup in grid order
 // instead of dealing the masked rows out took 31.1 us for the half-masked ones.

@@ -15,8 +15,8 @@ from kernels._native import host
 
 
 def _last_stride_1(x: Tensor) -> Tensor:
-    # the kernels need contiguous rows; other strides are fine
-    # (reference :113-115)
+    # the reference's helper (:113-115), kept for its callers; the calls below
+    # make rows readable natively (csrc/host_calls.cpp)
     return x if x.stride(-1) == 1 else x.contiguous()
 
 
