@@ -275,8 +275,17 @@ double prefill_us(int64_t bh, int32_t q_len, int32_t kv_len, int subs, int split
     partials += n > 1 ? n : 0;
   }
   const double cus = 256.0, mb = (double)(partials * bh) * 128 * bd3::kHeadDim * 8 / 1e6;
-  const double chain = c.chain0 + c.chain * longest;
+  double chain = c.chain0 + c.chain * longest;
   const double load = c.load0 + (c.load * (double)tiles + c.item * (double)items) * (double)bh / cus;
+  if (subs == 4 && items * bh > 256) {
+    // one workgroup a CU: the 257th item, longest first, follows another (2 x 12
+    // heads, 1463 queries over 4801 keys, 288 items: 73.6 us; 68.9 with two sets)
+    const auto item = [&](int64_t i) {
+      const int q1 = std::min(128 * ((q_len + 127) / 128 - (int)(i / bh)), q_len);
+      return c.chain0 + c.chain * (double)((kv_len - q_len + q1 + 63) / 64);
+    };
+    chain = std::max(chain, item(255) + item(256));
+  }
   const double walk = subs == 4 ? std::max(chain, load) : std::sqrt(chain * chain + load * load);
   return walk + (partials > 0 ? c.merge + c.partial * mb : 0.0);
 }
