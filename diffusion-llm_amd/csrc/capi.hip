@@ -338,9 +338,9 @@ double prefill_few_us(int64_t bh, int32_t q_len, int32_t kv_len, int subs, int s
 // 25.6 -> 18.3 (2), 8 x 512 (2 splits) 19.7 -> 12.9 (1); 2 x 200 queries over 4296 keys (11
 // splits) 21.3 -> 19.7 (2 sets, 5 splits), 1 x 136 over 2849 (12) 15.8 -> 13.6 (2, 8), 1 x
 // 71 over 799 (4) 10.2 as before (two sets without splits: 13.0). Over those 440
-// shapes 8% less time (geometric mean), 0.7% above the best plan of each; 366 others 9%
-// less, five of them 3-8% slower than with the earlier rule (one set was better
-// where the estimates of one and two differ by less than they err).
+// shapes 8% less time (geometric mean), 0.7% above the best plan of each; two of them are
+// more than 3% slower than with the earlier rule (5%), of 550 others, drawn over the
+// range and 11% faster, none more than 4%.
 PrefillPlan prefill_plan(int32_t batch, int32_t heads, int32_t q_len, int32_t kv_len, int32_t n_splits,
                          bool automatic) {
   constexpr int64_t kSplitItems = 128;
